@@ -46,6 +46,19 @@ def test_prefill_then_greedy_decode(gpu, oracle, model_dir, name, prompt_len, st
     assert_bits(gs.value_cache()[:, :pos], os_.value_cache()[:, :pos], "V cache")
 
 
+# gate/up tiles of 16, 32 and 64 tokens, their last and first batch, and the
+# GEMV's last
+@pytest.mark.parametrize("name", ["tiny", "tiny_q4", "tiny_pad"])
+@pytest.mark.parametrize("prompt_len", [7, 15, 16, 17, 32, 64, 65])
+def test_prefill_tile_edges(gpu, oracle, model_dir, name, prompt_len):
+    g, o, _ = _models(gpu, oracle, model_dir, name)
+    prompt = np.random.default_rng(prompt_len).integers(0, o.vocab, prompt_len).astype(np.uint32)
+    gs, os_ = g.create_session(), o.create_session()
+    assert_bits(g.forward_x(prompt, 0, gs), o.forward_x(prompt, 0, os_), "prefill logits")
+    assert_bits(gs.key_cache()[:, :prompt_len], os_.key_cache()[:, :prompt_len], "K cache")
+    assert_bits(gs.value_cache()[:, :prompt_len], os_.value_cache()[:, :prompt_len], "V cache")
+
+
 @pytest.mark.parametrize("name", ["tiny", "tiny_mixed", "tiny_yarn"])
 def test_generate_greedy_matches_oracle_tokens(gpu, oracle, model_dir, name):
     g, o, _ = _models(gpu, oracle, model_dir, name)

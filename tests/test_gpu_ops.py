@@ -176,6 +176,27 @@ def test_matmul_mfma_parity(gpu, oracle, fmt, batch, n, o):
     assert_bits(out, ref)
 
 
+# one case per tile configuration of the GEMM and per edge: a partial token and
+# row tile, odd block counts (rows' f16 scales start in either half of a
+# word), whole and partial stages of 4 blocks, fewer blocks than stages, and
+# the batches around where it takes over from the GEMV
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("batch,n,o", [(17, 96, 33), (40, 160, 65), (16, 32, 1), (16, 64, 97), (41, 1824, 190),
+                                       (100, 224, 4101), (130, 544, 5000), (400, 544, 4100), (1000, 96, 7300),
+                                       (4, 288, 14002), (4, 288, 4999), (13, 2048, 4400)])
+def test_matmul_mfma_tiles(gpu, oracle, fmt, batch, n, o):
+    from yallma3_mini_inference_amd import QuantizedWeight, WeightFormat, matmul
+    rng = np.random.default_rng(3 * n + o + batch + fmt)
+    wq = rng.integers(0, 16, o * n).astype(np.int8) if fmt else rng.integers(-128, 128, o * n).astype(np.int8)
+    ws = (rng.normal(0, 0.003, o * n // 32)).astype(np.float16).astype(np.float32)
+    w = QuantizedWeight.upload(WeightFormat(fmt), wq, ws, o, n)
+    xq, xs = oracle.quantize(fmt, rng.normal(0, 1, batch * n).astype(np.float32))
+    init = rng.normal(0, 1, batch * o).astype(np.float32)
+    out = matmul(init.copy(), xq, xs, w, n, o, fmt=WeightFormat(fmt))
+    ref = oracle.matmul_q8_slices(init.copy(), xq, xs, wq, ws, n, o)
+    assert_bits(out, ref)
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("negz", [False, True])
 @pytest.mark.parametrize("batch,n,o", [(96, 512, 384), (2048, 256, 2304)])

@@ -881,9 +881,12 @@ uint64_t gemv_bytes(const QMat& w, int out_elems, int batch) {
 // classes of yl_profile_kernel).
 enum OpClass : int { kOpQkv = 0, kOpAttn = 1, kOpWo = 2, kOpW13 = 3, kOpW2 = 4, kOpLogits = 5 };
 
-// Prompt batches from this many tokens run the projections on the int8
-// MFMA GEMM (activations normalized and quantized once per row first).
-constexpr int kGemmMinTokens = 16;
+// Prompt batches from this many tokens may run their projections on the int8
+// MFMA GEMM (activations normalized and quantized once per row first) where
+// gemm_preferred says so; the f32-scaled Q8 models, whose other path is the
+// tile kernel, always do from kGemmMinTokensQ8g on.
+constexpr int kGemmMinTokens = 8;
+constexpr int kGemmMinTokensQ8g = 4;
 
 // The projections of op `cls` of layer l over `batch` tokens on the GEMM
 // (prologue: the row normalization the QKV and gate/up GEMMs read first);
@@ -920,9 +923,14 @@ hipError_t enqueue_op_gemm(const yl_model* m, yl_session* s, int cls, int l, int
         return hipErrorNotSupported;
     }
     a.qs = w->qs; a.d = w->d; a.n = w->n; a.o = w->o; a.nb = w->nb;
-    if (!gemm_supported(a, w->fmt, epi, batch)) return hipErrorNotSupported;
+    // (the GEMV normalizes in its prologue, the GEMM behind a kernel of its
+    // own: half the rows count.  SmolLM2's 3072 gate/up rows at 8 tokens: a
+    // prompt of 1258 us with the GEMM, 1202 without)
+    const bool norm = cls == kOpQkv || cls == kOpW13;
+    if (!gemm_supported(a, w->fmt, epi, batch) || !gemm_preferred(w->fmt, norm ? w->o / 2 : w->o, batch))
+        return hipErrorNotSupported;
     hipError_t e = hipSuccess;
-    if (prologue && (cls == kOpQkv || cls == kOpW13)) {
+    if (prologue && norm) {
         // RMSNorm (+ the layer-0 embedding lookup) and quantization of every row
         if (cls == kOpQkv && l == 0) e = launch_embed(m->emb, tok, batch, s->x, st);
         if (e == hipSuccess)
@@ -958,6 +966,7 @@ hipError_t enqueue_op(const yl_model* m, yl_session* s, int cls, int l, int batc
     // several of the producers' 32-wide workgroups)
     const bool f32_act = m->q8g && m->gs > 32;
     if (batch >= kGemmMinTokens && cls != kOpAttn) {
+        // (hipErrorNotSupported also where the GEMV is the faster one)
         hipError_t e = enqueue_op_gemm(m, s, cls, l, batch, tok, kc, vc, bytes, prologue);
         if (e != hipErrorNotSupported) return e;
     }
@@ -1198,7 +1207,7 @@ hipError_t enqueue_op_q8g(const yl_model* m, yl_session* s, int cls, int l, int 
     const Layer& L = m->layers[l];
     float* kc = s->kc + (size_t)l * lay_kv;
     float* vc = s->vc + (size_t)l * lay_kv;
-    if (m->q8_gemv && batch >= kGemmMinTokens && cls != kOpAttn) {
+    if (m->q8_gemv && batch >= kGemmMinTokensQ8g && cls != kOpAttn) {
         const hipError_t e = enqueue_op_gemm_q8g(m, s, cls, l, batch, tok, kc, vc, bytes);
         if (e != hipErrorNotSupported) return e;
     }
@@ -1537,7 +1546,7 @@ yl_status yl_matmul(float* out, yl_format fmt, const int8_t* xq, const float* xs
     GemvArgs a{};
     a.qs = w->m.qs; a.d = w->m.d; a.n = w->m.n; a.o = w->m.o; a.nb = w->m.nb;
     a.xq = xq; a.xs = xs; a.out = out; a.accumulate_cols = (int)(o / 4 * 4);
-    const bool mfma = batch >= (size_t)kGemmMinTokens && gemm_supported(a, w->m.fmt, kEpiStore, (int)batch);
+    const bool mfma = gemm_preferred(w->m.fmt, (int)o, (int)batch) && gemm_supported(a, w->m.fmt, kEpiStore, (int)batch);
     const hipError_t e = mfma ? launch_gemm(a, w->m.fmt, kEpiStore, (int)batch, (hipStream_t)stream)
                               : launch_gemv(a, w->m.fmt, kEpiStore, (int)batch, (hipStream_t)stream);
     return e == hipSuccess ? YL_OK : hip_fail(e, "matmul launch");
@@ -1568,7 +1577,7 @@ yl_status yl_matmul_bench(const yl_weight* const* ws, size_t count, const int8_t
         GemvArgs a{};
         a.qs = w.qs; a.d = w.d; a.n = w.n; a.o = w.o; a.nb = w.nb;
         a.xq = xq; a.xs = xs; a.out = out; a.accumulate_cols = 0;
-        const bool mfma = batch >= (size_t)kGemmMinTokens && gemm_supported(a, w.fmt, kEpiStore, (int)batch);
+        const bool mfma = gemm_preferred(w.fmt, w.o, (int)batch) && gemm_supported(a, w.fmt, kEpiStore, (int)batch);
         ec = mfma ? launch_gemm(a, w.fmt, kEpiStore, (int)batch, st) : launch_gemv(a, w.fmt, kEpiStore, (int)batch, st);
     }
     if (e == hipSuccess) e = hipStreamEndCapture(st, &g);
