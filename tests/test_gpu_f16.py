@@ -38,6 +38,20 @@ def _pair(oracle, model_dir, name):
     return Transformer(path), oracle.Model(path)
 
 
+# one case per tile of the batched kernel (by its number of outputs), with
+# partial row, token and column tiles, and both sides of the first bound
+@pytest.mark.parametrize("o,n,batch", [(33, 32, 2), (17, 96, 17), (6400, 32, 16), (6401, 32, 16), (3001, 160, 33),
+                                       (8191, 64, 90), (7001, 96, 433)])
+def test_matmul_f32_batch_tiles(gpu, oracle, o, n, batch):
+    from yallma3_mini_inference_amd.weight_type import QuantizedWeight, matmul_f32
+    rng = np.random.default_rng(o + n + batch)
+    w16 = (rng.standard_normal((o, n)) * 0.05).astype(np.float16)
+    x = rng.standard_normal((batch, n)).astype(np.float32)
+    ref = np.zeros((batch, o), np.float32)
+    oracle.matmul_f32(ref, x, w16.astype(np.float32), n, o)
+    assert_bits(matmul_f32(x, QuantizedWeight.upload_f16(w16, o, n), n, o), ref, "matmul_f32")
+
+
 @pytest.mark.parametrize("name,prompt_len,steps", [("tiny_f16", 20, 16), ("tiny_f16", 100, 4),
                                                     ("tiny_q8_f16emb", 20, 8), ("tiny_q8_f16emb", 90, 3),
                                                     ("small_f16", 70, 6)])

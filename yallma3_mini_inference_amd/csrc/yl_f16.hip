@@ -350,101 +350,145 @@ __global__ void k_swiglu_pairs(const float* __restrict__ raw, int hidden, float*
 }
 
 // --------------------------------------------------------------- batches
-// A workgroup owns 64 rows x 64 tokens: lane r of wavefront w runs the
-// chains of row r for the 16 tokens 16w .. 16w+15, one accumulator each, so
-// every weight tile is read once per 64 tokens.  Per K tile of 32 columns
-// the weights ([64 rows][32 halves], row stride 80 bytes) and the
-// activations ([32 columns][64 tokens] f32, read as broadcast vf4 of 4
-// tokens) sit in LDS, double-buffered; the next tile's global loads are in
-// registers while the current tile is added.  Each chain adds its products
-// x[t][k] * w[r][k] in column order (matmul_f32's serial sum).
-constexpr int kFbRows = 64;          // rows per workgroup (lane = row)
-constexpr int kFbTok = 64;           // tokens per workgroup (16 per wavefront)
-constexpr int kFbKT = 32;            // columns per tile
-constexpr int kFbWStride = 40;       // halves per weight row in LDS (32 + 8: 16-byte aligned, spread banks)
-constexpr int kFbXStride = kFbTok + 4;   // floats per activation column in LDS
+// A lane runs the chains of RR rows x CC tokens, one accumulator each; the
+// 64 lanes of a wavefront are (64 / TL) row lanes x TL token lanes, and the
+// four wavefronts lie WT along the tokens, 4 / WT along the rows.  Per K
+// tile of 64 columns the weights (halves, [row][k]) and the activations (f32,
+// [token][k]) sit in LDS, double-buffered; the next tile's global loads are
+// in registers while the current tile is added.  Rows are padded so that the
+// 16-byte reads of the row (token) lanes fall on distinct banks.  Each chain
+// adds its products x[t][k] * w[r][k] in column order (matmul_f32's serial
+// sum).
+// Bound: two f32 operations per product (the product and the sum are rounded
+// apart) plus one widening per RR = 1 row and column, and, while the chip is
+// not full, the chain of n dependent sums.  So few outputs take one chain
+// per lane and many take 4 x 4, which read each LDS word for 4 products.
+constexpr int kFbKT = 64;            // columns per tile (32: 3 to 10% slower)
 
-template <int EPI>
+template <int RR, int CC, int TL, int WT>
+struct FbShape {
+    static constexpr int ws = kFbKT + 8, xs = kFbKT + 4;   // row strides in LDS: halves per weight row, floats per token
+    static constexpr int RL = 64 / TL, WR = 4 / WT;
+    static constexpr int rows = WR * RL * RR, toks = WT * TL * CC;
+    // 16-byte pieces per thread and tile
+    static constexpr int wp = rows * (kFbKT / 8), xp = toks * (kFbKT / 4);
+    static constexpr int wn = (wp + 255) / 256, xn = (xp + 255) / 256;
+};
+
+template <int EPI, int RR, int CC, int TL, int WT>
 __global__ __launch_bounds__(256) void k_matmul_f16_batch(const uint16_t* __restrict__ w, int n, int o,
                                                           const float* __restrict__ x, int batch,
                                                           float* __restrict__ out, int out_ld) {
-    __shared__ __align__(16) uint16_t wt[2][kFbRows * kFbWStride];
-    __shared__ __align__(16) float xt[2][kFbKT * kFbXStride];
+    using S = FbShape<RR, CC, TL, WT>;
+    __shared__ __align__(16) uint16_t wt[2][S::rows * S::ws];
+    __shared__ __align__(16) float xt[2][S::toks * S::xs];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int row0 = blockIdx.x * kFbRows, tok0 = blockIdx.y * kFbTok;
+    const int row0 = blockIdx.x * S::rows, tok0 = blockIdx.y * S::toks;
     const int ntile = (n + kFbKT - 1) / kFbKT;
-    // loader thread i: weight chunk (row i / 4, halves 8 (i % 4) .. +8); two
-    // activation float4 (token i / 4 ... see below)
-    const int wr_row = tid >> 2, wr_c = (tid & 3) * 8;
-    uint4 wreg;
-    vf4 xreg[2];
+    // piece i of a tile: row (token) i / pieces-per-row; rows, tokens and
+    // columns past the matrix re-read its last ones (unused)
+    uint4 wreg[S::wn];
+    vf4 xreg[S::xn];
     auto load = [&](int t) {
         const int k0 = t * kFbKT;
-        const int r = min(row0 + wr_row, o - 1);
-        wreg = *reinterpret_cast<const uint4*>(w + (size_t)r * n + min(k0 + wr_c, n - 8));
-        // activations: 64 tokens x 32 columns = 512 float4; thread i takes
-        // float4 i and i + 256: token (j / 8), columns 4 (j % 8) .. +3
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int j = tid + 256 * h;
-            const int tk = min(tok0 + (j >> 3), batch - 1);
-            xreg[h] = *reinterpret_cast<const vf4*>(x + (size_t)tk * n + min(k0 + 4 * (j & 7), n - 4));
+        for (int h = 0; h < S::wn; h++) {
+            const int i = tid + 256 * h, r = min(row0 + i / (kFbKT / 8), o - 1);
+            if (S::wp % 256 == 0 || i < S::wp)
+                wreg[h] = *reinterpret_cast<const uint4*>(w + (size_t)r * n + min(k0 + 8 * (i % (kFbKT / 8)), n - 8));
+        }
+#pragma unroll
+        for (int h = 0; h < S::xn; h++) {
+            const int i = tid + 256 * h, tk = min(tok0 + i / (kFbKT / 4), batch - 1);
+            if (S::xp % 256 == 0 || i < S::xp)
+                xreg[h] = *reinterpret_cast<const vf4*>(x + (size_t)tk * n + min(k0 + 4 * (i % (kFbKT / 4)), n - 4));
         }
     };
     auto store = [&](int b) {
-        *reinterpret_cast<uint4*>(&wt[b][wr_row * kFbWStride + wr_c]) = wreg;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int j = tid + 256 * h;
-            const int tk = j >> 3, c = 4 * (j & 7);
-            xt[b][(c + 0) * kFbXStride + tk] = xreg[h].x;
-            xt[b][(c + 1) * kFbXStride + tk] = xreg[h].y;
-            xt[b][(c + 2) * kFbXStride + tk] = xreg[h].z;
-            xt[b][(c + 3) * kFbXStride + tk] = xreg[h].w;
+        for (int h = 0; h < S::wn; h++) {
+            const int i = tid + 256 * h;
+            if (S::wp % 256 == 0 || i < S::wp)
+                *reinterpret_cast<uint4*>(&wt[b][i / (kFbKT / 8) * S::ws + 8 * (i % (kFbKT / 8))]) = wreg[h];
+        }
+#pragma unroll
+        for (int h = 0; h < S::xn; h++) {
+            const int i = tid + 256 * h;
+            if (S::xp % 256 == 0 || i < S::xp)
+                *reinterpret_cast<vf4*>(&xt[b][i / (kFbKT / 4) * S::xs + 4 * (i % (kFbKT / 4))]) = xreg[h];
         }
     };
+    // this lane's rows rl + RL * r and tokens tl + TL * c of its wavefront's block
+    const int rl = (wave % S::WR) * S::RL * RR + lane / TL, tl = (wave / S::WR) * TL * CC + lane % TL;
     load(0);
     store(0);
     __syncthreads();
-    float acc[16];
+    float acc[RR][CC];
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+    for (int r = 0; r < RR; r++)
+#pragma unroll
+        for (int c = 0; c < CC; c++) acc[r][c] = 0.0f;
     for (int t = 0; t < ntile; t++) {
         const int b = t & 1;
         if (t + 1 < ntile) load(t + 1);
-        const int kn = min(kFbKT, n - t * kFbKT);   // 32, or 32 (n % 32 == 0)
-        const uint16_t* wrow = &wt[b][lane * kFbWStride];
-        const float* xc = &xt[b][16 * wave];
+        const int kn = min(kFbKT, n - t * kFbKT);   // kFbKT, or 32 (n % 32 == 0)
+        // 8 columns, their operands read while the previous 8 are added
+        uint4 wq[2][RR];
+        vf4 xq[2][CC][2];
+        auto read = [&](int c8, uint4 (&wv)[RR], vf4 (&xv)[CC][2]) {
+#pragma unroll
+            for (int r = 0; r < RR; r++)
+                wv[r] = *reinterpret_cast<const uint4*>(&wt[b][(rl + S::RL * r) * S::ws + 8 * c8]);
+#pragma unroll
+            for (int c = 0; c < CC; c++)
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    xv[c][i] = *reinterpret_cast<const vf4*>(&xt[b][(tl + TL * c) * S::xs + 8 * c8 + 4 * i]);
+        };
+        read(0, wq[0], xq[0]);
 #pragma unroll
         for (int c8 = 0; c8 < kFbKT / 8; c8++) {
             if (8 * c8 >= kn) break;
-            float wf[8];
-            widen8(*reinterpret_cast<const uint4*>(wrow + 8 * c8), wf);
+            if (c8 + 1 < kFbKT / 8) read(c8 + 1, wq[(c8 + 1) & 1], xq[(c8 + 1) & 1]);
+            float wf[RR][8];
 #pragma unroll
-            for (int kk = 0; kk < 8; kk++) {
-                const float* xk = xc + (8 * c8 + kk) * kFbXStride;
-                const vf4 x0 = *reinterpret_cast<const vf4*>(xk), x1 = *reinterpret_cast<const vf4*>(xk + 4),
-                          x2 = *reinterpret_cast<const vf4*>(xk + 8), x3 = *reinterpret_cast<const vf4*>(xk + 12);
-                const float xs[16] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w,
-                                      x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
+            for (int r = 0; r < RR; r++) widen8(wq[c8 & 1][r], wf[r]);
+            // the products of PK columns, then their sums: no sum waits on a
+            // product just issued
+            constexpr int PK = RR * CC >= 4 ? 2 : 8;
 #pragma unroll
-                for (int i = 0; i < 16; i++) acc[i] = fadd(acc[i], fmul(xs[i], wf[kk]));
+            for (int k1 = 0; k1 < 8; k1 += PK) {
+                float p[PK][RR][CC];
+#pragma unroll
+                for (int kk = 0; kk < PK; kk++)
+#pragma unroll
+                    for (int r = 0; r < RR; r++)
+#pragma unroll
+                        for (int c = 0; c < CC; c++)
+                            p[kk][r][c] = fmul(xq[c8 & 1][c][(k1 + kk) / 4][(k1 + kk) % 4], wf[r][k1 + kk]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int kk = 0; kk < PK; kk++)
+#pragma unroll
+                    for (int r = 0; r < RR; r++)
+#pragma unroll
+                        for (int c = 0; c < CC; c++) acc[r][c] = fadd(acc[r][c], p[kk][r][c]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (t + 1 < ntile) store(b ^ 1);
         __syncthreads();
     }
-    const int row = row0 + lane;
-    if (row < o) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int tk = tok0 + 16 * wave + i;
-            if (tk < batch) {
+    for (int r = 0; r < RR; r++)
+#pragma unroll
+        for (int c = 0; c < CC; c++) {
+            const int row = row0 + rl + S::RL * r, tk = tok0 + tl + TL * c;
+            if (row < o && tk < batch) {
                 float* dst = out + (size_t)tk * out_ld + row;
-                *dst = EPI == 0 ? acc[i] : fadd(*dst, acc[i]);
+                *dst = EPI == 0 ? acc[r][c] : fadd(*dst, acc[r][c]);
             }
         }
-    }
 }
 
 // ------------------------------------------------------------------ QKV
@@ -489,14 +533,34 @@ __global__ void k_qkv_f16(const float* __restrict__ raw, const float* __restrict
     }
 }
 
+template <int RR, int CC, int TL, int WT>
+static hipError_t launch_fb(const uint16_t* w, int n, int o, const float* x, int batch, float* out, int out_ld, int epi,
+                            hipStream_t s) {
+    using S = FbShape<RR, CC, TL, WT>;
+    auto k = epi == 0 ? k_matmul_f16_batch<0, RR, CC, TL, WT> : k_matmul_f16_batch<1, RR, CC, TL, WT>;
+    hipLaunchKernelGGL(k, dim3((o + S::rows - 1) / S::rows, (batch + S::toks - 1) / S::toks), dim3(256), 0, s, w, n, o, x,
+                       batch, out, out_ld);
+    return hipGetLastError();
+}
+
 hipError_t launch_matmul_f16(const uint16_t* w, int n, int o, const float* x, int batch, float* out, int out_ld,
                              int epi, hipStream_t s) {
     if (n % 32 || n <= 0 || o <= 0 || batch <= 0 || epi < 0 || epi > 1) return hipErrorInvalidValue;
     if (batch == 1) return launch_f16_gemv(w, n, o, x, nullptr, 0.0f, epi, out, s);
-    const int rb = (o + kFbRows - 1) / kFbRows;
-    auto k = epi == 0 ? k_matmul_f16_batch<0> : k_matmul_f16_batch<1>;
-    hipLaunchKernelGGL(k, dim3(rb, (batch + kFbTok - 1) / kFbTok), dim3(256), 0, s, w, n, o, x, batch, out, out_ld);
-    return hipGetLastError();
+    const long outs = (long)o * batch;
+    // Measured (us; 64 rows x 64 tokens per workgroup, 16 chains per lane
+    // before; rows x columns, tokens):
+    //                     1x1     1x2     1x4     2x4    before
+    //   2048 x 2048, 8    24.9    34.4    52      88      205
+    //   2048 x 2048, 48   29.4    35.3    53.9    87      205
+    //   2048 x 2048, 190  65      57      70      91      206
+    //   3072 x 2048, 300  138     120     112     113     207
+    //   2048 x 8192, 512  562     459     428     442     820
+    //   8000 x 2048, 512  538     437     401     372     373
+    if (outs <= 102400) return launch_fb<1, 1, 8, 2>(w, n, o, x, batch, out, out_ld, epi, s);
+    if (outs <= 512000) return launch_fb<1, 2, 8, 2>(w, n, o, x, batch, out, out_ld, epi, s);
+    if (outs <= 3000000) return launch_fb<1, 4, 4, 2>(w, n, o, x, batch, out, out_ld, epi, s);
+    return launch_fb<2, 4, 4, 4>(w, n, o, x, batch, out, out_ld, epi, s);
 }
 
 template <int PRO, int EPI, int R>
