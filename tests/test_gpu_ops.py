@@ -345,6 +345,24 @@ def test_attention(gpu, oracle, batch, start, nh, nkv, hd):
     assert_bits(out, ref)
 
 
+# batches below the tiled path: one, two and four rows per workgroup (by the
+# grid), partial row groups, odd and short contexts, every head size class
+@pytest.mark.parametrize("batch,start,nh,nkv,hd", [(2, 0, 4, 2, 64), (3, 5, 9, 3, 64), (16, 1, 32, 8, 64),
+                                                   (17, 30, 32, 8, 64), (31, 100, 32, 8, 128), (33, 2, 32, 8, 64),
+                                                   (45, 1200, 32, 8, 64), (63, 0, 16, 16, 32), (29, 12, 32, 4, 40),
+                                                   (58, 3, 9, 3, 64), (5, 3700, 64, 8, 64)])
+def test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd):
+    from yallma3_mini_inference_amd import ops
+    rng = np.random.default_rng(batch * 1000 + start)
+    seq = start + batch
+    q = rng.normal(0, 1, batch * nh * hd).astype(np.float32)
+    kc = rng.normal(0, 1, seq * nkv * hd).astype(np.float32)
+    vc = rng.normal(0, 1, seq * nkv * hd).astype(np.float32)
+    scale = float(np.float32(1.0) / np.sqrt(np.float32(hd)))
+    out = ops.attention(q, kc, vc, batch, start, nh, nkv, hd, scale)
+    assert_bits(out, oracle.fused_attention(q, kc, vc, seq, batch, nh, nkv, hd, start, nkv * hd, scale))
+
+
 # One-token contexts around the register P.V chains' bounds: 1 to 7 registers
 # of 16 chunks (8 positions each), partial registers, a seq % 8 tail or none,
 # 112 chunks (the most held in registers) and the LDS-tile chains past it.

@@ -8,8 +8,8 @@
 //
 // k_attn_decode (one token): grid (n_heads, head_size/32), one workgroup
 // per 32 output dimensions of a head, independent of every other
-// workgroup.  k_attention (prompt batches) keeps one workgroup per
-// (head, token) with the causal mask of the whole call's span.
+// workgroup.  k_attention (prompt batches) takes one to four tokens of a
+// head per workgroup, with the causal mask of the whole call's span.
 #include <hip/hip_runtime.h>
 
 #include "yl_blocks.h"
@@ -19,19 +19,6 @@
 namespace yl {
 
 constexpr int kAttnThreads = 256;
-
-template <int QF>
-__device__ void quantize_head_output(const float* outl, int hd, int8_t* aq, float* as, size_t group0) {
-    const int ng = hd / kGroup;
-    for (int g = threadIdx.x; g < ng; g += blockDim.x) {
-        const float* v = outl + g * kGroup;
-        float amax = 0.0f;
-        for (int k = 0; k < kGroup; k++) amax = fmaxf(amax, fabsf(v[k]));
-        const float s = group_scale<QF>(amax);
-        as[group0 + g] = s;
-        for (int k = 0; k < kGroup; k++) aq[(group0 + g) * kGroup + k] = (int8_t)quant_one<QF>(v[k], s);
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Decode (one token).  Workgroup (h, ds) owns query head h and the 32
@@ -904,11 +891,43 @@ __global__ __launch_bounds__(HD) void k_attn_pv_out(const float* __restrict__ vc
 }
 
 // ---------------------------------------------------------------------------
-// Prompt batches: one workgroup per (query head, token); seq_len = pos +
-// batch, the token's own position pos + t, later positions masked to -1e10.
-// LDS: scores seq_len | q head_size | partials 8*head_size | out head_size.
+// Prompt batches: one workgroup per (query head, R consecutive tokens);
+// seq_len = pos + batch, token t's own position pos + t, later positions
+// masked to -1e10.  Every K and V value is read once for the R rows (one row
+// per workgroup: 920 MB from L2 for 45 tokens at 1200 positions, 32 heads of
+// 64).  R is 1, 2 or 4: the most that leaves a workgroup per CU, and 1 below
+// 256 positions, where a workgroup is a few latencies long.  Measured, us for
+// R = 1 / 2 / 4 (the kernel with one row, scalar key loads and the sum and
+// quantization on single threads before):
+//   45 tokens from 1200, 32 heads of 64    57.5 / 46.3 / 44.5   (53.9)
+//   60 tokens from 1300, 32 heads of 128   156 / 106 / 75       (122)
+//   41 tokens from 0, 32 heads of 64       7.6 / 8.4 / 10.6     (14.0)
+// At 1245 positions a workgroup of 4 rows spends 30 K cycles on scores and
+// 25 K on P.V (L2 round trips, two or one block ahead) and 18 K on the sums.
+//   1. scores: a thread computes 2 positions x R rows (8-byte key loads, q as
+//      scalars), written as sc[position][R];
+//   2. row maxima, exponentials, the R serial sums side by side in R lanes
+//      of wavefront 0, p = e / sum;
+//   3. P.V: a thread runs the chains of lane j, 2 dimensions and R rows, its
+//      R p values one broadcast LDS read;
+//   4. reduce_add8, the seq % 8 tail, the quantized groups.
+// LDS (floats): sc seq_len * R | partials R * 8 * head_size | reduction.
 // ---------------------------------------------------------------------------
-template <int QF>
+typedef float vf2u __attribute__((ext_vector_type(2), aligned(4)));   // two floats at any float address
+template <int R>
+struct VecR { typedef float t __attribute__((ext_vector_type(R))); };
+
+static __host__ __device__ inline int attention_sc_floats(int seq_len, int rows) { return ((seq_len + 15) & ~15) * rows; }
+
+// s + lanes 0..15 of the caller's 16-lane row of v, one at a time
+template <int K>
+__device__ __forceinline__ float add_row_lanes(float s, float v) {
+    s = fadd(row_bcast_lane<K>(v), s);
+    if constexpr (K < 15) s = add_row_lanes<K + 1>(s, v);
+    return s;
+}
+
+template <int QF, int R>
 __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restrict__ sq,
                                                             const float* __restrict__ kc,
                                                             const float* __restrict__ vc,
@@ -918,110 +937,254 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
                                                             float* __restrict__ as,
                                                             float* __restrict__ att_f32) {
     extern __shared__ __align__(16) float lds_f[];
-    __shared__ float red[8];
-    const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
+    __shared__ float red[kAttnThreads / 64][R];
+    __shared__ float inv_sh[R];
+    constexpr int PP = R == 1 ? 1 : 2;   // positions per thread and round
+    typedef typename VecR<R>::t vr;
+    typedef typename VecR<PP>::t vp;
+    constexpr int NW = kAttnThreads / 64;
+    const int h = blockIdx.x, t0 = blockIdx.y * R, tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pos0 = st->pos;
     const int seq_len = pos0 + batch;
-    const int abs_pos = pos0 + t;
-    const int max_t2 = abs_pos < seq_len - 1 ? abs_pos : seq_len - 1;
     const int kvh = h / (n_heads / n_kv_heads);
     const int kv_dim = n_kv_heads * hd;
     const int att_dim = n_heads * hd;
-    float* sc = lds_f;
-    float* ql = sc + ((seq_len + 3) & ~3);
-    float* part = ql + hd;
-    float* outl = part + 8 * hd;
+    vr* sc = reinterpret_cast<vr*>(lds_f);
+    float* part = lds_f + attention_sc_floats(seq_len, R);
 
-    for (int i = tid; i < hd; i += kAttnThreads) ql[i] = sq[(size_t)t * att_dim + (size_t)h * hd + i];
-    __syncthreads();
-    float lmax = -1e10f;
-    const int n_simd = hd / 8;
-    for (int t2 = tid; t2 <= max_t2; t2 += kAttnThreads) {
-        // keys transposed: dimension i of position t2 at kt[i * kv_ld]
-        const float* kt = kc + (size_t)kvh * hd * kv_ld + t2;
-        float l[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int s = 0; s < n_simd; s++) {
-            const float* q = ql + s * 8;
+    // 1. scores (rows past the batch repeat its last token, unused)
+    const float* q[R];
 #pragma unroll
-            for (int j = 0; j < 8; j++) l[j] = fadd(l[j], fmul(q[j], kt[(size_t)(8 * s + j) * kv_ld]));
+    for (int r = 0; r < R; r++) q[r] = sq + (size_t)min(t0 + r, batch - 1) * att_dim + (size_t)h * hd;
+    float lmax[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) lmax[r] = -1e10f;
+    const int last = min(pos0 + t0 + R - 1, seq_len - 1);   // the rows' last causal position
+    const int n_simd = hd / 8;
+    for (int t2 = PP * tid; t2 < seq_len; t2 += PP * kAttnThreads) {
+        vr v[PP];
+        if (t2 <= last) {
+            // keys transposed: dimension i of position t2 at kt[i * kv_ld]
+            // (kv_ld is even); the loads of 16 dimensions are in flight
+            const float* kt = kc + (size_t)kvh * hd * kv_ld + t2;
+            float l[R][PP][8];
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int b = 0; b < PP; b++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) l[r][b][j] = 0.0f;
+            vp kn[2][8];
+            auto load_k = [&](vp (&k)[8], int s) {
+                const float* ks = kt + (size_t)(8 * min(s, n_simd - 1)) * kv_ld;
+#pragma unroll
+                for (int j = 0; j < 8; j++) k[j] = *reinterpret_cast<const vp*>(ks + (size_t)j * kv_ld);
+            };
+            auto step = [&](vp (&k)[8], int s) {
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const float qv = q[r][8 * s + j];
+#pragma unroll
+                        for (int b = 0; b < PP; b++) l[r][b][j] = fadd(l[r][b][j], fmul(qv, k[j][b]));
+                    }
+                load_k(k, s + 2);
+            };
+            load_k(kn[0], 0);
+            load_k(kn[1], 1);
+#pragma unroll 1
+            for (int s = 0; s + 1 < n_simd; s += 2) {
+                step(kn[0], s);
+                step(kn[1], s + 1);
+            }
+            if (n_simd & 1) step(kn[0], n_simd - 1);
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int b = 0; b < PP; b++) {
+                    const bool live = t2 + b <= min(pos0 + t0 + r, seq_len - 1);
+                    const float sv = live ? fmul(reduce_add8(l[r][b]), attn_scale) : -1e10f;
+                    if (live) lmax[r] = fmaxf(lmax[r], sv);
+                    v[b][r] = sv;
+                }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++)
+#pragma unroll
+                for (int b = 0; b < PP; b++) v[b][r] = -1e10f;
         }
-        const float sv = fmul(reduce_add8(l), attn_scale);
-        sc[t2] = sv;
-        lmax = fmaxf(lmax, sv);
+#pragma unroll
+        for (int b = 0; b < PP; b++) sc[t2 + b] = v[b];   // (the row is padded past an odd length)
     }
-    for (int t2 = max_t2 + 1 + tid; t2 < seq_len; t2 += kAttnThreads) sc[t2] = -1e10f;
-    lmax = wave_max(lmax);
-    if ((tid & 63) == 0) red[tid >> 6] = lmax;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        lmax[r] = wave_max(lmax[r]);
+        if ((tid & 63) == 0) red[wave][r] = lmax[r];
+    }
     __syncthreads();
-    float mx = red[0];
-    for (int w = 1; w < kAttnThreads / 64; w++) mx = fmaxf(mx, red[w]);
-    for (int t2 = tid; t2 < seq_len; t2 += kAttnThreads) sc[t2] = expf_rn(sc[t2] - mx);
+    // 2. exponentials, sums, probabilities
+    float mx[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        mx[r] = red[0][r];
+#pragma unroll
+        for (int w = 1; w < NW; w++) mx[r] = fmaxf(mx[r], red[w][r]);
+    }
+    const ExpfK ek = expf_k_regs();
+    for (int t2 = tid; t2 < ((seq_len + 15) & ~15); t2 += kAttnThreads) {
+        vr e = sc[t2];
+#pragma unroll
+        for (int r = 0; r < R; r++) e[r] = t2 < seq_len ? expf_rn(e[r] - mx[r], ek) : 0.0f;
+        sc[t2] = e;
+    }
     __syncthreads();
-    if (tid == 0) {
+    // the R serial sums side by side: lanes 16r .. 16r + 15 of wavefront 0
+    // hold 16 consecutive e of row r, and each adds its 16-lane row's values
+    // one at a time (DPP broadcasts); the row is +0 up to a multiple of 16
+    if (wave == 0) {
+        const int r = (tid >> 4) & (R - 1);
+        const float* e = lds_f + (tid & 15) * R + r;
+        const int n16 = (seq_len + 15) / 16;
         float sum = 0.0f;
-        int t2 = 0;
-        for (; t2 + 4 <= seq_len; t2 += 4) {
-            const float4 e4 = *reinterpret_cast<const float4*>(sc + t2);
-            sum = fadd(sum, e4.x);
-            sum = fadd(sum, e4.y);
-            sum = fadd(sum, e4.z);
-            sum = fadd(sum, e4.w);
+        float nx[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) nx[i] = e[min(i, n16 - 1) * 16 * R];
+        for (int m = 0; m < n16; m += 4) {
+            float cur[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                cur[i] = m + i < n16 ? nx[i] : 0.0f;
+                nx[i] = e[min(m + 4 + i, n16 - 1) * 16 * R];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) sum = add_row_lanes<0>(sum, cur[i]);
         }
-        for (; t2 < seq_len; t2++) sum = fadd(sum, sc[t2]);
-        red[4] = sum > 0.0f ? 1.0f / sum : 0.0f;
+        if ((tid & 15) == 0 && tid < 16 * R) inv_sh[r] = sum > 0.0f ? 1.0f / sum : 0.0f;
     }
     __syncthreads();
-    const float inv = red[4];
-    for (int t2 = tid; t2 < seq_len; t2 += kAttnThreads) sc[t2] = fmul(sc[t2], inv);
+    float inv[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) inv[r] = inv_sh[r];
+    for (int t2 = tid; t2 < seq_len; t2 += kAttnThreads) {
+        vr e = sc[t2];
+#pragma unroll
+        for (int r = 0; r < R; r++) e[r] = fmul(e[r], inv[r]);
+        sc[t2] = e;
+    }
     __syncthreads();
-    const int n_chunks = seq_len / 8;
+    // 3. chains of lane j, dimensions 2 d2 and 2 d2 + 1
+    const int n_chunks = seq_len / 8, half = hd / 2;
     const float* vbase = vc + (size_t)kvh * hd;
-    for (int ch = tid; ch < 8 * hd; ch += kAttnThreads) {
-        const int d = ch % hd, j = ch / hd;
-        float l = 0.0f;
-        const float* vp = vbase + (size_t)j * kv_dim + d;
-#pragma unroll 8
-        for (int cc = 0; cc < n_chunks; cc++) l = fadd(l, fmul(sc[8 * cc + j], vp[(size_t)(8 * cc) * kv_dim]));
-        part[j * hd + d] = l;
+    for (int ch = tid; ch < 8 * half; ch += kAttnThreads) {
+        const int d2 = ch % half, j = ch / half;
+        float l[R][2];
+#pragma unroll
+        for (int r = 0; r < R; r++) l[r][0] = l[r][1] = 0.0f;
+        const float* vp2 = vbase + (size_t)j * kv_dim + 2 * d2;
+        const vr* pp = sc + j;
+        // blocks of 8 chunks, the next block's V in flight
+        vf2u va[8], vb[8];
+        auto load_v = [&](vf2u (&v)[8], int c0) {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                v[i] = *reinterpret_cast<const vf2u*>(vp2 + (size_t)(8 * min(c0 + i, n_chunks - 1)) * kv_dim);
+        };
+        auto add_v = [&](const vf2u (&v)[8], int c0, int n) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                if (i >= n) break;
+                const vr p = pp[8 * (c0 + i)];
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    l[r][0] = fadd(l[r][0], fmul(p[r], v[i].x));
+                    l[r][1] = fadd(l[r][1], fmul(p[r], v[i].y));
+                }
+            }
+        };
+        if (n_chunks > 0) load_v(va, 0);
+        int c0 = 0;
+#pragma unroll 1
+        for (; c0 + 16 <= n_chunks; c0 += 16) {
+            load_v(vb, c0 + 8);
+            add_v(va, c0, 8);
+            load_v(va, c0 + 16);
+            add_v(vb, c0 + 8, 8);
+        }
+        if (c0 + 8 < n_chunks) load_v(vb, c0 + 8);
+        add_v(va, c0, n_chunks - c0);
+        add_v(vb, c0 + 8, n_chunks - c0 - 8);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            part[(r * 8 + j) * hd + 2 * d2] = l[r][0];
+            part[(r * 8 + j) * hd + 2 * d2 + 1] = l[r][1];
+        }
     }
     __syncthreads();
-    for (int d = tid; d < hd; d += kAttnThreads) {
+    // 4. outputs, one per thread (whole wavefronts of lanes: the group
+    // maxima below need every lane)
+    const int n_out = R * hd;
+    for (int i0 = 0; i0 < n_out; i0 += kAttnThreads) {
+        const int i = min(i0 + tid, n_out - 1), r = i / hd, d = i % hd, t = t0 + r;
+        const bool live = i0 + tid < n_out && t < batch;
         float l[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) l[j] = part[j * hd + d];
+        for (int j = 0; j < 8; j++) l[j] = part[(r * 8 + j) * hd + d];
         float sum = reduce_add8(l);
         for (int t2 = n_chunks * 8; t2 < seq_len; t2++)
-            sum = fadd(sum, fmul(sc[t2], vbase[(size_t)t2 * kv_dim + d]));
-        outl[d] = sum;
-        if (att_f32) att_f32[(size_t)t * att_dim + (size_t)h * hd + d] = sum;
+            sum = fadd(sum, fmul(lds_f[t2 * R + r], vbase[(size_t)t2 * kv_dim + d]));
+        const size_t col = (size_t)t * att_dim + (size_t)h * hd + d;
+        if (att_f32 && live) att_f32[col] = sum;
+        if constexpr (QF >= 0) {
+            const float am = fmaxf(group_max(fabsf(sum), 32), 0.0f);
+            const float s = group_scale<QF>(am);
+            if (live) {
+                aq[col] = (int8_t)quant_one<QF>(sum, s);
+                if ((d & 31) == 0) as[col / kGroup] = s;
+            }
+        }
     }
-    __syncthreads();
-    if constexpr (QF >= 0)
-        quantize_head_output<QF>(outl, hd, aq, as, (size_t)t * (att_dim / kGroup) + ((size_t)h * hd) / kGroup);
 }
 
-static size_t attention_lds_bytes(int seq_len, int head_size) {
-    return ((size_t)((seq_len + 3) & ~3) + 10 * (size_t)head_size) * sizeof(float);
+static size_t attention_lds_bytes(int seq_len, int head_size, int rows) {
+    return ((size_t)attention_sc_floats(seq_len, rows) + 8 * (size_t)rows * head_size) * sizeof(float);
 }
-bool attention_row_fits(int seq_len, int head_size) { return attention_lds_bytes(seq_len, head_size) <= 60 * 1024; }
+// (a property of the call: the one-row form's score row, q, partials and
+// output within 60 KiB)
+bool attention_row_fits(int seq_len, int head_size) {
+    return ((size_t)((seq_len + 3) & ~3) + 10 * (size_t)head_size) * sizeof(float) <= 60 * 1024;
+}
+
+template <int QF>
+static hipError_t launch_attention_q(const float* sq, const float* kc, const float* vc, const StepState* st, int batch,
+                                     int max_seq, int kv_ld, int n_heads, int n_kv_heads, int head_size, float scale,
+                                     int8_t* aq, float* as, float* att_f32, hipStream_t s) {
+    auto go = [&](auto k, int rows) {
+        hipLaunchKernelGGL(k, dim3(n_heads, (batch + rows - 1) / rows), dim3(kAttnThreads),
+                           attention_lds_bytes(max_seq, head_size, rows), s, sq, kc, vc, st, batch, kv_ld, n_heads,
+                           n_kv_heads, head_size, scale, aq, as, att_f32);
+        return hipGetLastError();
+    };
+    auto rows_ok = [&](int rows) {
+        return max_seq >= 256 && (long)n_heads * ((batch + rows - 1) / rows) >= 256 &&
+               attention_lds_bytes(max_seq, head_size, rows) <= 60 * 1024;
+    };
+    if (rows_ok(4)) return go(k_attention<QF, 4>, 4);
+    if (rows_ok(2)) return go(k_attention<QF, 2>, 2);
+    return go(k_attention<QF, 1>, 1);
+}
 
 hipError_t launch_attention(const float* sq, const float* kc, const float* vc, const StepState* st, int batch,
                             int max_seq, int kv_ld, int n_heads, int n_kv_heads, int head_size, float scale, int qfmt,
                             int8_t* aq, float* as, float* att_f32, hipStream_t s) {
-    // max_seq: the seq_len of this call (LDS holds its score row)
-    if (!attention_row_fits(max_seq, head_size)) return hipErrorInvalidValue;
-    const size_t smem = attention_lds_bytes(max_seq, head_size);
-    const dim3 grid(n_heads, batch);
+    // max_seq: the seq_len of this call (LDS holds its score rows)
+    if (!attention_row_fits(max_seq, head_size) || kv_ld % 2 || head_size % 8) return hipErrorInvalidValue;
     if (qfmt == kQ8)
-        hipLaunchKernelGGL((k_attention<kQ8>), grid, dim3(kAttnThreads), smem, s, sq, kc, vc, st, batch, kv_ld,
-                           n_heads, n_kv_heads, head_size, scale, aq, as, att_f32);
-    else if (qfmt == kQ4)
-        hipLaunchKernelGGL((k_attention<kQ4>), grid, dim3(kAttnThreads), smem, s, sq, kc, vc, st, batch, kv_ld,
-                           n_heads, n_kv_heads, head_size, scale, aq, as, att_f32);
-    else
-        hipLaunchKernelGGL((k_attention<-1>), grid, dim3(kAttnThreads), smem, s, sq, kc, vc, st, batch, kv_ld,
-                           n_heads, n_kv_heads, head_size, scale, aq, as, att_f32);
-    return hipGetLastError();
+        return launch_attention_q<kQ8>(sq, kc, vc, st, batch, max_seq, kv_ld, n_heads, n_kv_heads, head_size, scale, aq, as, att_f32, s);
+    if (qfmt == kQ4)
+        return launch_attention_q<kQ4>(sq, kc, vc, st, batch, max_seq, kv_ld, n_heads, n_kv_heads, head_size, scale, aq, as, att_f32, s);
+    return launch_attention_q<-1>(sq, kc, vc, st, batch, max_seq, kv_ld, n_heads, n_kv_heads, head_size, scale, aq, as, att_f32, s);
 }
 
 size_t attn_decode_lds_bytes(int max_seq) { return attn_decode_lds_floats(max_seq) * sizeof(float); }
