@@ -417,6 +417,37 @@ def test_swiglu_quantize(gpu, oracle, hidden, batch, qfmt):
         assert_bits(s, os_)
 
 
+# ends of the row kernels' chunks and passes: less than a workgroup, one, two
+# and four passes, a partial last one; rows without quantized output of any
+# length (elements past the last whole 8 come out zero)
+@pytest.mark.parametrize("size,batch,qfmt", [(32, 3, 0), (2080, 2, 1), (4128, 2, 0), (8192, 2, 1), (8, 2, -1),
+                                             (30, 3, -1), (2061, 2, -1)])
+def test_row_kernel_edges(gpu, oracle, size, batch, qfmt):
+    from yallma3_mini_inference_amd import WeightFormat, ops, quantize
+    rng = np.random.default_rng(size + batch)
+    x = rng.normal(0, 2, (batch, size)).astype(np.float32)
+    u = rng.normal(0, 1, (batch, size)).astype(np.float32)
+    w = rng.normal(1, 0.2, size).astype(np.float32)
+    n8 = size // 8 * 8
+    ref = np.zeros((batch, size), np.float32)
+    for t in range(batch):
+        ref[t] = oracle.rmsnorm(x[t], w, 1e-5) if n8 == size else 0.0
+    xn, q, s = ops.rmsnorm_quantize(x, w, 1e-5, qfmt)
+    if n8 == size:
+        assert_bits(xn, ref)
+    else:
+        assert np.all(xn[:, n8:] == 0) and np.all(np.isfinite(xn))
+    h, hq, hs = ops.swiglu_quantize(x, u, qfmt)
+    href = np.stack([oracle.swiglu(x[t], u[t]) for t in range(batch)])
+    if n8 == size:
+        assert_bits(h, href)
+    if qfmt >= 0:
+        for got, want in (((q, s), ref), ((hq, hs), href), (quantize(WeightFormat(qfmt), x.ravel()), x)):
+            oq, os_ = oracle.quantize(qfmt, want.ravel())
+            np.testing.assert_array_equal(np.asarray(got[0]).ravel(), oq)
+            assert_bits(got[1], os_)
+
+
 def test_serial_sum_exact(gpu):
     # the softmax denominator's serial sum by one wavefront (forward.rs:356-361)
     import sys, os

@@ -111,20 +111,20 @@ __device__ __forceinline__ int quant_one(float x, float scale) {
     return q;
 }
 
-// quant_one over 8 values of one group, without a division per value.
+// quant_one over N (8, or 4) values of one group, without a division per value.
 // y = x * fl(1/scale) is within |x/scale| * 2^-23 <= 2^-16 of x/scale (the
 // quotient never exceeds 127 * (1 + 2^-23) in magnitude), and so is the
 // reference's fl(x/scale).  When y lies more than 2^-14 from every
 // half-integer, both round to rint(y); otherwise (and for NaN, an infinite
 // or zero reciprocal, or a scale below 2^-100) the lane takes quant_one's
 // exact division.  Ties therefore always go through the exact path.
-template <int FMT>
-__device__ __forceinline__ void quant8(const float v[8], float scale, int q[8]) {
+template <int FMT, int N = 8>
+__device__ __forceinline__ void quant8(const float v[N], float scale, int q[N]) {
     const float rinv = 1.0f / scale;
     bool slow = !(rinv <= 0x1p100f);
     constexpr float lo = FMT == kQ4 ? -7.0f : -128.0f, hi = FMT == kQ4 ? 7.0f : 127.0f;
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < N; k++) {
         const float y = v[k] * rinv;
         const float r = __builtin_rintf(y);
         slow = slow || !(__builtin_fabsf(y - r) <= 0.5f - 0x1p-14f);
@@ -132,7 +132,7 @@ __device__ __forceinline__ void quant8(const float v[8], float scale, int q[8]) 
     }
     if (slow) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) q[k] = quant_one<FMT>(v[k], scale);
+        for (int k = 0; k < N; k++) q[k] = quant_one<FMT>(v[k], scale);
     }
 }
 
