@@ -363,6 +363,15 @@ def test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd):
     assert_bits(out, oracle.fused_attention(q, kc, vc, seq, batch, nh, nkv, hd, start, nkv * hd, scale))
 
 
+# the tiled path's side of its bound with k_attention (heads x tokens x head
+# size above 2^20, or a score row too long for four in LDS) and the last call
+# below it
+@pytest.mark.parametrize("batch,start,nh,nkv,hd", [(129, 0, 64, 8, 128), (128, 0, 64, 8, 128), (520, 5, 32, 4, 64),
+                                                   (70, 3400, 4, 2, 64), (64, 3200, 4, 2, 64), (1030, 0, 32, 32, 32)])
+def test_attention_tiled_bound(gpu, oracle, batch, start, nh, nkv, hd):
+    test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd)
+
+
 # One-token contexts around the register P.V chains' bounds: 1 to 7 registers
 # of 16 chunks (8 positions each), partial registers, a seq % 8 tail or none,
 # 112 chunks (the most held in registers) and the LDS-tile chains past it.
@@ -397,6 +406,23 @@ def test_prompt_attention_nonfinite_v(gpu, oracle):
     scale = float(np.float32(1.0) / np.sqrt(np.float32(hd)))
     out = ops.attention(q, kc, vc, batch, start, nh, nkv, hd, scale)
     ref = oracle.fused_attention(q, kc, vc, seq, batch, nh, nkv, hd, start, nkv * hd, scale)
+    nan = np.isnan(ref)
+    assert nan.any() and np.array_equal(np.isnan(out), nan)
+    assert_bits(out[~nan], ref[~nan])
+
+
+def test_tiled_attention_nonfinite_v(gpu, oracle):
+    # the same on a call large enough for the tiled kernels
+    from yallma3_mini_inference_amd import ops
+    batch, start, nh, nkv, hd = 260, 10, 64, 4, 64
+    rng = np.random.default_rng(260)
+    seq = start + batch
+    q = rng.normal(0, 1, batch * nh * hd).astype(np.float32)
+    kc = rng.normal(0, 1, seq * nkv * hd).astype(np.float32)
+    vc = rng.normal(0, 1, seq * nkv * hd).astype(np.float32)
+    vc[(start + 250) * nkv * hd + 3] = np.inf
+    out = ops.attention(q, kc, vc, batch, start, nh, nkv, hd, 0.125)
+    ref = oracle.fused_attention(q, kc, vc, seq, batch, nh, nkv, hd, start, nkv * hd, 0.125)
     nan = np.isnan(ref)
     assert nan.any() and np.array_equal(np.isnan(out), nan)
     assert_bits(out[~nan], ref[~nan])

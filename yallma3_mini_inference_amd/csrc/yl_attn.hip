@@ -1156,6 +1156,10 @@ bool attention_row_fits(int seq_len, int head_size) {
     return ((size_t)((seq_len + 3) & ~3) + 10 * (size_t)head_size) * sizeof(float) <= 60 * 1024;
 }
 
+bool attention_rows4_fit(int seq_len, int head_size) {
+    return attention_row_fits(seq_len, head_size) && attention_lds_bytes(seq_len, head_size, 4) <= 60 * 1024;
+}
+
 template <int QF>
 static hipError_t launch_attention_q(const float* sq, const float* kc, const float* vc, const StepState* st, int batch,
                                      int max_seq, int kv_ld, int n_heads, int n_kv_heads, int head_size, float scale,

@@ -168,6 +168,8 @@ hipError_t launch_embed(const EmbQ8& e, const uint32_t* tokens, int batch, float
 // kc: keys [kv_dim][kv_ld] (transposed), vc: values [max_seq][kv_dim];
 // max_seq = the call's seq_len, which attention_row_fits() must accept
 bool attention_row_fits(int seq_len, int head_size);
+// four such rows fit one workgroup
+bool attention_rows4_fit(int seq_len, int head_size);
 hipError_t launch_attention(const float* sq, const float* kc, const float* vc, const StepState* st,
                             int batch, int max_seq, int kv_ld, int n_heads, int n_kv_heads, int head_size,
                             float scale, int qfmt, int8_t* aq, float* as, float* att_f32,
@@ -186,6 +188,7 @@ hipError_t launch_attn_decode(const float* sq, const float* kc, const float* vc,
 // too long for k_attention's LDS row: tiled attention over a scratch of
 // prompt_attn_bytes(n_heads, seq_len, batch); seq_ld = pos + batch (host side)
 bool prompt_attn_applies(int batch, int seq_len, int head_size);
+bool prompt_attn_tiled(int batch, int seq_len, int n_heads, int head_size);
 size_t prompt_attn_bytes(int n_heads, int seq_ld, int batch);
 hipError_t launch_prompt_attention(const float* sq, const float* kc, const float* vc, const StepState* st, int batch,
                                    int seq_ld, int kv_ld, int n_heads, int n_kv_heads, int head_size, float scale,

@@ -806,7 +806,7 @@ yl_model* model_from_host(HostModel& h, yl_status* st) {
 // the largest size used; prompts below 64 tokens need none).
 bool prompt_scratch(yl_session* s, int batch, uint32_t start_pos) {
     s->pseq = (int)start_pos + batch;
-    if (!prompt_attn_applies(batch, s->pseq, s->m->hd)) return true;
+    if (!prompt_attn_tiled(batch, s->pseq, s->m->n_heads, s->m->hd)) return true;
     const size_t need = prompt_attn_bytes(s->m->n_heads, s->pseq, batch);
     if (need <= s->psc_bytes) return true;
     hipStreamSynchronize(s->stream);
@@ -1001,7 +1001,7 @@ hipError_t enqueue_op(const yl_model* m, yl_session* s, int cls, int l, int batc
         if (batch == 1)
             return launch_attn_decode(s->sq, kc, vc, s->st, s->dec_seq, m->kv_ld, m->n_heads, m->n_kv, m->hd,
                                       m->attn_scale, L.wo.fmt, s->aq, s->as_, nullptr, s->sc, st);
-        if (prompt_attn_applies(batch, s->pseq, m->hd))
+        if (prompt_attn_tiled(batch, s->pseq, m->n_heads, m->hd))
             return launch_prompt_attention(s->sq, kc, vc, s->st, batch, s->pseq, m->kv_ld, m->n_heads, m->n_kv, m->hd,
                                            m->attn_scale, L.wo.fmt, s->aq, s->as_, nullptr, s->psc, st);
         return launch_attention(s->sq, kc, vc, s->st, batch, s->pseq, m->kv_ld, m->n_heads, m->n_kv, m->hd,
@@ -1051,7 +1051,7 @@ static hipError_t enqueue_attn_f32(const yl_model* m, yl_session* s, int batch, 
     if (batch == 1)
         return launch_attn_decode(s->sq, kc, vc, s->st, s->dec_seq, m->kv_ld, m->n_heads, m->n_kv, m->hd,
                                   m->attn_scale, -1, nullptr, nullptr, s->attf, s->sc, st);
-    if (prompt_attn_applies(batch, s->pseq, m->hd))
+    if (prompt_attn_tiled(batch, s->pseq, m->n_heads, m->hd))
         return launch_prompt_attention(s->sq, kc, vc, s->st, batch, s->pseq, m->kv_ld, m->n_heads, m->n_kv, m->hd,
                                        m->attn_scale, -1, nullptr, nullptr, s->attf, s->psc, st);
     return launch_attention(s->sq, kc, vc, s->st, batch, s->pseq, m->kv_ld, m->n_heads, m->n_kv, m->hd,
@@ -1691,7 +1691,7 @@ hipError_t attention_enqueue(float* out, const float* q, const float* kc, const 
     if (batch == 1)
         return launch_attn_decode(q, kt, vc, dst, seq, B.ld, (int)n_heads, (int)n_kv_heads, (int)hd, attn_scale, -1,
                                   nullptr, nullptr, out, sc, strm);
-    if (sc)
+    if (prompt_attn_tiled((int)batch, seq, (int)n_heads, (int)hd))
         return launch_prompt_attention(q, kt, vc, dst, (int)batch, seq, B.ld, (int)n_heads, (int)n_kv_heads, (int)hd,
                                        attn_scale, -1, nullptr, nullptr, out, sc, strm);
     return launch_attention(q, kt, vc, dst, (int)batch, seq, B.ld, (int)n_heads, (int)n_kv_heads, (int)hd,

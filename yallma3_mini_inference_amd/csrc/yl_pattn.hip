@@ -57,11 +57,24 @@ size_t prompt_attn_bytes(int n_heads, int seq_ld, int batch) {
     const size_t Bp = pattn_rows_ld(batch);
     return (size_t)n_heads * Bp * ((size_t)seq_ld + pattn_tiles(seq_ld) + 3) * sizeof(float);
 }
-// k_attention (one workgroup per head and token) holds the whole score row
-// in LDS; batches of 2..63 tokens whose seq_len does not fit take the tiled
-// path as one partial row tile
+// Calls that the tiled path was sized for (and whose scratch a caller must
+// have): 64 tokens or more, and shorter ones whose score row does not fit
+// k_attention's LDS.
 bool prompt_attn_applies(int batch, int seq_len, int head_size) {
     return batch >= kPT || (batch > 1 && !attention_row_fits(seq_len, head_size));
+}
+// Of those, the ones that run on it: it needs enough (head, 64-row tile)
+// workgroups to fill the chip, since each walks its positions serially, while
+// k_attention re-reads K and V once per 4 rows.  They meet at heads x tokens x
+// head size of about 2^20.  Whole prompts, tiled against k_attention: 1B shape
+// (32 heads of 64) 128 tokens 4.90 / 1.92 ms, 512 5.36 / 4.77, 700 6.91 /
+// 6.86, 1000 8.62 / 10.1; SmolLM2 (9 heads of 64) 512 tokens 5.44 / 2.52,
+// 1400 10.4 / 7.86, 2000 14.5 / 12.9.  64 tokens onto 1200, 32 heads of 64:
+// 242 / 48.8 us.
+bool prompt_attn_tiled(int batch, int seq_len, int n_heads, int head_size) {
+    if (!prompt_attn_applies(batch, seq_len, head_size)) return false;
+    if (head_size != 32 && head_size != 64 && head_size != 128) return true;   // (refused there)
+    return !attention_rows4_fit(seq_len, head_size) || (long)batch * n_heads * head_size > (1l << 20);
 }
 
 // ---------------------------------------------------------------------------
