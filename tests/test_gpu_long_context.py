@@ -107,6 +107,17 @@ def test_decode_bound_of_head_size_32(gpu, oracle, model_dir):
     assert_bits(g.forward_x(prompt, P + 1, gs), o.forward_x(prompt, P + 1, os_), "prompt at 16384")
 
 
+@pytest.mark.parametrize("prompt_len", [300, 323])
+def test_prompt_row_groups_quantized_head_size_32(gpu, oracle, model_dir, prompt_len):
+    """Head size 32 with the quantized output on two and four rows per
+    workgroup (4 heads, 1200 and 1292 rows in all)."""
+    g, o, _ = _models(oracle, model_dir, "tiny_hd32_long")
+    gs, os_ = g.create_session(), o.create_session()
+    prompt = np.random.default_rng(prompt_len).integers(0, o.vocab, prompt_len).astype(np.uint32)
+    assert_bits(g.forward_x(prompt, 0, gs), o.forward_x(prompt, 0, os_), "prompt")
+    assert_bits(gs.value_cache()[:, :prompt_len], os_.value_cache()[:, :prompt_len], "V cache")
+
+
 def test_split_decode_attention_in_graph(gpu, oracle, model_dir):
     """ctx 8448 (bucket 8448): decode at 5000+ runs k_attn_scores, softmax,
     P.V by lane and the output kernel inside the decode graph with seq well

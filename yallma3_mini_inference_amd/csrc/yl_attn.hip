@@ -12,6 +12,8 @@
 // head per workgroup, with the causal mask of the whole call's span.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "yl_blocks.h"
 #include "yl_device.h"
 #include "yl_internal.h"
@@ -895,27 +897,33 @@ __global__ __launch_bounds__(HD) void k_attn_pv_out(const float* __restrict__ vc
 // seq_len = pos + batch, token t's own position pos + t, later positions
 // masked to -1e10.  Every K and V value is read once for the R rows (one row
 // per workgroup: 920 MB from L2 for 45 tokens at 1200 positions, 32 heads of
-// 64).  R is 1, 2 or 4: the most that leaves a workgroup per CU, and 1 below
-// 256 positions, where a workgroup is a few latencies long.  Measured, us for
-// R = 1 / 2 / 4 (the kernel with one row, scalar key loads and the sum and
-// quantization on single threads before):
-//   45 tokens from 1200, 32 heads of 64    57.5 / 46.3 / 44.5   (53.9)
-//   60 tokens from 1300, 32 heads of 128   156 / 106 / 75       (122)
-//   41 tokens from 0, 32 heads of 64       7.6 / 8.4 / 10.6     (14.0)
+// 64).  R is 1, 2 or 4 (attention_rows).  Measured, us (a workgroup per row,
+// scalar key loads and the quantization on single threads before):
+//   45 tokens from 1200, 32 heads of 64    44.0  (54.1)
+//   60 tokens from 1300, 32 heads of 128   75    (131)
+//   41 tokens from 0, 32 heads of 64       7.6   (8.5; 14.0 quantized)
+//   2 tokens from 1300, 9 heads of 64      26.8  (35.8)
+// The smallest calls at head sizes 8 to 32 are bound by instruction fetch:
+// 2 to 9 tokens from 0 with an f32 output take 4.9 us (4.5 before, in half
+// the code).
 // At 1245 positions a workgroup of 4 rows spends 30 K cycles on scores and
 // 25 K on P.V (L2 round trips, two or one block ahead) and 18 K on the sums.
 //   1. scores: a thread computes 2 positions x R rows (8-byte key loads, q as
-//      scalars), written as sc[position][R];
-//   2. row maxima, exponentials, the R serial sums side by side in R lanes
-//      of wavefront 0, p = e / sum;
-//   3. P.V: a thread runs the chains of lane j, 2 dimensions and R rows, its
-//      R p values one broadcast LDS read;
+//      scalars; one position if R = 1), written as sc[position][R];
+//   2. row maxima, exponentials, the R serial sums side by side in 16-lane
+//      rows of wavefront 0 (one row: plain adds of broadcast reads, 6 us less
+//      than the DPP adds at 3200 positions), p = e / sum;
+//   3. P.V: a thread runs the chains of lane j, DD dimensions and R rows, its
+//      R p values one broadcast LDS read.  DD = 2, or 1 where 8 x head_size
+//      chains are at most one round of threads (with 2 half of them idle: 16
+//      tokens from 1200, 32 heads of 32, 24.7 us against 20.0);
 //   4. reduce_add8, the seq % 8 tail, the quantized groups.
 // LDS (floats): sc seq_len * R | partials R * 8 * head_size | reduction.
 // ---------------------------------------------------------------------------
-typedef float vf2u __attribute__((ext_vector_type(2), aligned(4)));   // two floats at any float address
 template <int R>
 struct VecR { typedef float t __attribute__((ext_vector_type(R))); };
+template <int D>
+struct VecU { typedef float t __attribute__((ext_vector_type(D), aligned(4))); };   // D floats at any float address
 
 static __host__ __device__ inline int attention_sc_floats(int seq_len, int rows) { return ((seq_len + 15) & ~15) * rows; }
 
@@ -927,7 +935,7 @@ __device__ __forceinline__ float add_row_lanes(float s, float v) {
     return s;
 }
 
-template <int QF, int R>
+template <int QF, int R, int DD>
 __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restrict__ sq,
                                                             const float* __restrict__ kc,
                                                             const float* __restrict__ vc,
@@ -977,7 +985,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
                     for (int j = 0; j < 8; j++) l[r][b][j] = 0.0f;
             vp kn[2][8];
             auto load_k = [&](vp (&k)[8], int s) {
-                const float* ks = kt + (size_t)(8 * min(s, n_simd - 1)) * kv_ld;
+                const float* ks = kt + (size_t)(8 * s) * kv_ld;
 #pragma unroll
                 for (int j = 0; j < 8; j++) k[j] = *reinterpret_cast<const vp*>(ks + (size_t)j * kv_ld);
             };
@@ -990,16 +998,27 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
 #pragma unroll
                         for (int b = 0; b < PP; b++) l[r][b][j] = fadd(l[r][b][j], fmul(qv, k[j][b]));
                     }
-                load_k(k, s + 2);
             };
             load_k(kn[0], 0);
-            load_k(kn[1], 1);
+            if (n_simd > 1) load_k(kn[1], 1);
+            int s = 0;
 #pragma unroll 1
-            for (int s = 0; s + 1 < n_simd; s += 2) {
+            for (; s + 3 < n_simd; s += 2) {
                 step(kn[0], s);
+                load_k(kn[0], s + 2);
                 step(kn[1], s + 1);
+                load_k(kn[1], s + 3);
             }
-            if (n_simd & 1) step(kn[0], n_simd - 1);
+            // the last 1 to 3 (no load past the head: at head size 8 such
+            // re-reads were two loads of three)
+            if (s + 2 < n_simd) {
+                step(kn[0], s);
+                load_k(kn[0], s + 2);
+                step(kn[1], s + 1);
+                s += 2;
+            }
+            step(kn[0], s);
+            if (s + 1 < n_simd) step(kn[1], s + 1);
 #pragma unroll
             for (int r = 0; r < R; r++)
 #pragma unroll
@@ -1043,7 +1062,25 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
     // the R serial sums side by side: lanes 16r .. 16r + 15 of wavefront 0
     // hold 16 consecutive e of row r, and each adds its 16-lane row's values
     // one at a time (DPP broadcasts); the row is +0 up to a multiple of 16
-    if (wave == 0) {
+    if (wave == 0 && R == 1) {
+        const vf4* e4 = reinterpret_cast<const vf4*>(lds_f);
+        const int n16 = (seq_len + 15) / 16;
+        float sum = 0.0f;
+        vf4 nx[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) nx[i] = e4[i];
+        for (int m = 0; m < n16; m++) {
+            vf4 cur[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                cur[i] = nx[i];
+                nx[i] = e4[4 * min(m + 1, n16 - 1) + i];
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) sum = fadd(sum, cur[i / 4][i % 4]);
+        }
+        if (tid == 0) inv_sh[0] = sum > 0.0f ? 1.0f / sum : 0.0f;
+    } else if (wave == 0) {
         const int r = (tid >> 4) & (R - 1);
         const float* e = lds_f + (tid & 15) * R + r;
         const int n16 = (seq_len + 15) / 16;
@@ -1051,16 +1088,20 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
         float nx[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) nx[i] = e[min(i, n16 - 1) * 16 * R];
-        for (int m = 0; m < n16; m += 4) {
+        int m = 0;
+        for (; m + 4 <= n16; m += 4) {
             float cur[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                cur[i] = m + i < n16 ? nx[i] : 0.0f;
+                cur[i] = nx[i];
                 nx[i] = e[min(m + 4 + i, n16 - 1) * 16 * R];
             }
 #pragma unroll
             for (int i = 0; i < 4; i++) sum = add_row_lanes<0>(sum, cur[i]);
         }
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (m + i < n16) sum = add_row_lanes<0>(sum, nx[i]);
         if ((tid & 15) == 0 && tid < 16 * R) inv_sh[r] = sum > 0.0f ? 1.0f / sum : 0.0f;
     }
     __syncthreads();
@@ -1074,33 +1115,35 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
         sc[t2] = e;
     }
     __syncthreads();
-    // 3. chains of lane j, dimensions 2 d2 and 2 d2 + 1
-    const int n_chunks = seq_len / 8, half = hd / 2;
+    // 3. chains of lane j, dimensions DD * dq .. + DD - 1
+    typedef typename VecU<DD>::t vd;
+    const int n_chunks = seq_len / 8, nd = hd / DD;
     const float* vbase = vc + (size_t)kvh * hd;
-    for (int ch = tid; ch < 8 * half; ch += kAttnThreads) {
-        const int d2 = ch % half, j = ch / half;
-        float l[R][2];
+    for (int ch = tid; ch < 8 * nd; ch += kAttnThreads) {
+        const int dq = ch % nd, j = ch / nd;
+        float l[R][DD];
 #pragma unroll
-        for (int r = 0; r < R; r++) l[r][0] = l[r][1] = 0.0f;
-        const float* vp2 = vbase + (size_t)j * kv_dim + 2 * d2;
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int k = 0; k < DD; k++) l[r][k] = 0.0f;
+        const float* vpd = vbase + (size_t)j * kv_dim + DD * dq;
         const vr* pp = sc + j;
         // blocks of 8 chunks, the next block's V in flight
-        vf2u va[8], vb[8];
-        auto load_v = [&](vf2u (&v)[8], int c0) {
+        vd va[8], vb[8];
+        auto load_v = [&](vd (&v)[8], int c0) {
 #pragma unroll
             for (int i = 0; i < 8; i++)
-                v[i] = *reinterpret_cast<const vf2u*>(vp2 + (size_t)(8 * min(c0 + i, n_chunks - 1)) * kv_dim);
+                v[i] = *reinterpret_cast<const vd*>(vpd + (size_t)(8 * min(c0 + i, n_chunks - 1)) * kv_dim);
         };
-        auto add_v = [&](const vf2u (&v)[8], int c0, int n) {
+        auto add_v = [&](const vd (&v)[8], int c0, int n) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 if (i >= n) break;
                 const vr p = pp[8 * (c0 + i)];
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    l[r][0] = fadd(l[r][0], fmul(p[r], v[i].x));
-                    l[r][1] = fadd(l[r][1], fmul(p[r], v[i].y));
-                }
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int k = 0; k < DD; k++) l[r][k] = fadd(l[r][k], fmul(p[r], v[i][k]));
             }
         };
         if (n_chunks > 0) load_v(va, 0);
@@ -1116,17 +1159,16 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
         add_v(va, c0, n_chunks - c0);
         add_v(vb, c0 + 8, n_chunks - c0 - 8);
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            part[(r * 8 + j) * hd + 2 * d2] = l[r][0];
-            part[(r * 8 + j) * hd + 2 * d2 + 1] = l[r][1];
-        }
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int k = 0; k < DD; k++) part[(r * 8 + j) * hd + DD * dq + k] = l[r][k];
     }
     __syncthreads();
     // 4. outputs, one per thread (whole wavefronts of lanes: the group
     // maxima below need every lane)
     const int n_out = R * hd;
     for (int i0 = 0; i0 < n_out; i0 += kAttnThreads) {
-        const int i = min(i0 + tid, n_out - 1), r = i / hd, d = i % hd, t = t0 + r;
+        const int i = min(i0 + tid, n_out - 1), r = R == 1 ? 0 : i / hd, d = i - r * hd, t = t0 + r;
         const bool live = i0 + tid < n_out && t < batch;
         float l[8];
 #pragma unroll
@@ -1156,8 +1198,34 @@ bool attention_row_fits(int seq_len, int head_size) {
     return ((size_t)((seq_len + 3) & ~3) + 10 * (size_t)head_size) * sizeof(float) <= 60 * 1024;
 }
 
-bool attention_rows4_fit(int seq_len, int head_size) {
-    return attention_row_fits(seq_len, head_size) && attention_lds_bytes(seq_len, head_size, 4) <= 60 * 1024;
+int attention_rows_fit(int seq_len, int head_size) {
+    if (!attention_row_fits(seq_len, head_size)) return 0;
+    int rows = 4;
+    while (rows > 1 && attention_lds_bytes(seq_len, head_size, rows) > 60 * 1024) rows /= 2;
+    return rows;
+}
+// Rows per workgroup, by rows in all (n = n_heads * batch).  One-row
+// workgroups read K and V once per row but run seven or eight to a CU (64 or
+// 65 registers, against 110 to 127): while all n run at once on short
+// contexts, one row is the fastest.  From 256 positions the reads weigh more
+// than the latencies and two rows are faster from two one-row workgroups per
+// CU on (four at head size 32, where a row's chains are half as long), four
+// from five.  Measured, us for 1 / 2 / 4 rows:
+//   n 1056, head size 64,  183 positions   10.6 / 11.4 / 13.2
+//   n 1536, head size 128, 198             20.1 / 17.1 / 18.6
+//   n 2016, head size 64,  63               8.5 /  9.0 / 10.5
+//   n 2112, head size 128, 183             24.8 / 28.0 / 20.8
+//   n 288,  head size 64,  1232            24.9 / 28.7 / 36.5
+//   n 1056, head size 64,  1232            45.2 / 40.0 / 41.6
+//   n 2112, head size 64,  1232            76.4 / 69.6 / 50.8
+//   n 512,  head size 32,  1215            20.0 / 22.1 / 26.3
+//   n 1056, head size 32,  1232            30.8 / 28.8 / 30.2
+static int attention_rows(int batch, int seq_len, int n_heads, int head_size) {
+    const long n = (long)n_heads * batch;
+    int rows;
+    if (seq_len < 256) rows = n > 2048 ? 4 : (n > 1792 || (n >= 1536 && seq_len >= 128) ? 2 : 1);
+    else rows = n >= 1280 ? 4 : (n >= (head_size <= 32 ? 1024 : 512) ? 2 : 1);
+    return std::min(rows, attention_rows_fit(seq_len, head_size));
 }
 
 template <int QF>
@@ -1170,13 +1238,15 @@ static hipError_t launch_attention_q(const float* sq, const float* kc, const flo
                            n_kv_heads, head_size, scale, aq, as, att_f32);
         return hipGetLastError();
     };
-    auto rows_ok = [&](int rows) {
-        return max_seq >= 256 && (long)n_heads * ((batch + rows - 1) / rows) >= 256 &&
-               attention_lds_bytes(max_seq, head_size, rows) <= 60 * 1024;
-    };
-    if (rows_ok(4)) return go(k_attention<QF, 4>, 4);
-    if (rows_ok(2)) return go(k_attention<QF, 2>, 2);
-    return go(k_attention<QF, 1>, 1);
+    const int rows = attention_rows(batch, max_seq, n_heads, head_size);
+    if (head_size <= kAttnThreads / 8) {   // (8 lanes x head_size chains are one round of threads)
+        if (rows == 4) return go(k_attention<QF, 4, 1>, 4);
+        if (rows == 2) return go(k_attention<QF, 2, 1>, 2);
+        return go(k_attention<QF, 1, 1>, 1);
+    }
+    if (rows == 4) return go(k_attention<QF, 4, 2>, 4);
+    if (rows == 2) return go(k_attention<QF, 2, 2>, 2);
+    return go(k_attention<QF, 1, 2>, 1);
 }
 
 hipError_t launch_attention(const float* sq, const float* kc, const float* vc, const StepState* st, int batch,

@@ -74,7 +74,7 @@ bool prompt_attn_applies(int batch, int seq_len, int head_size) {
 bool prompt_attn_tiled(int batch, int seq_len, int n_heads, int head_size) {
     if (!prompt_attn_applies(batch, seq_len, head_size)) return false;
     if (head_size != 32 && head_size != 64 && head_size != 128) return true;   // (refused there)
-    return !attention_rows4_fit(seq_len, head_size) || (long)batch * n_heads * head_size > (1l << 20);
+    return attention_rows_fit(seq_len, head_size) < 4 || (long)batch * n_heads * head_size > (1l << 20);
 }
 
 // ---------------------------------------------------------------------------
