@@ -376,12 +376,25 @@ def test_attention_row_groups(gpu, oracle, batch, start, nh, nkv, hd):
     test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd)
 
 
-# the tiled path's side of its bound with k_attention (heads x tokens x head
-# size above 2^20, or a score row too long for four in LDS) and the last call
-# below it
+# calls of 64 tokens or more on the tiled path and on k_attention, with whole
+# and partial row tiles
 @pytest.mark.parametrize("batch,start,nh,nkv,hd", [(129, 0, 64, 8, 128), (128, 0, 64, 8, 128), (520, 5, 32, 4, 64),
                                                    (70, 3400, 4, 2, 64), (64, 3200, 4, 2, 64), (1030, 0, 32, 32, 32)])
 def test_attention_tiled_bound(gpu, oracle, batch, start, nh, nkv, hd):
+    test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd)
+
+
+# the last call on k_attention and the first on the tiled path, per head size
+# and by what a CU's LDS holds: three 4-row workgroups (the last context of
+# them at head size 64), two, 2-row workgroups, none
+@pytest.mark.parametrize("batch,start,nh,nkv,hd", [(768, 0, 32, 4, 32), (769, 0, 32, 4, 32), (320, 7, 64, 8, 64),
+                                                   (321, 7, 64, 8, 64), (192, 3, 64, 8, 128), (193, 3, 64, 8, 128),
+                                                   (192, 2624, 64, 8, 64), (193, 2623, 64, 8, 64), (193, 2624, 64, 8, 64),
+                                                   (128, 2200, 64, 8, 128), (129, 2200, 64, 8, 128),
+                                                   (256, 3010, 64, 8, 32), (257, 3010, 64, 8, 32),
+                                                   (128, 3230, 64, 8, 64), (129, 3230, 64, 8, 64),
+                                                   (64, 7104, 2, 1, 64), (64, 7105, 2, 1, 64)])
+def test_attention_tiled_bounds_by_head_size(gpu, oracle, batch, start, nh, nkv, hd):
     test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd)
 
 

@@ -1204,6 +1204,11 @@ int attention_rows_fit(int seq_len, int head_size) {
     while (rows > 1 && attention_lds_bytes(seq_len, head_size, rows) > 60 * 1024) rows /= 2;
     return rows;
 }
+// (a CU's 160 KiB hold three workgroups of at most 42 pieces of 1280 bytes)
+bool attention_rows4_three_per_cu(int seq_len, int head_size) {
+    return attention_lds_bytes(seq_len, head_size, 4) <= 52 * 1024;
+}
+
 // Rows per workgroup, by rows in all (n = n_heads * batch).  One-row
 // workgroups read K and V once per row but run seven or eight to a CU (64 or
 // 65 registers, against 110 to 127): while all n run at once on short

@@ -168,8 +168,10 @@ hipError_t launch_embed(const EmbQ8& e, const uint32_t* tokens, int batch, float
 // kc: keys [kv_dim][kv_ld] (transposed), vc: values [max_seq][kv_dim];
 // max_seq = the call's seq_len, which attention_row_fits() must accept
 bool attention_row_fits(int seq_len, int head_size);
-// how many such rows (0, 1, 2 or 4) fit one workgroup
+// how many such rows (0, 1, 2 or 4) fit one workgroup, and whether three
+// workgroups of four fit a CU's LDS
 int attention_rows_fit(int seq_len, int head_size);
+bool attention_rows4_three_per_cu(int seq_len, int head_size);
 hipError_t launch_attention(const float* sq, const float* kc, const float* vc, const StepState* st,
                             int batch, int max_seq, int kv_ld, int n_heads, int n_kv_heads, int head_size,
                             float scale, int qfmt, int8_t* aq, float* as, float* att_f32,

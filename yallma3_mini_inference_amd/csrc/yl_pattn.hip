@@ -63,18 +63,31 @@ size_t prompt_attn_bytes(int n_heads, int seq_ld, int batch) {
 bool prompt_attn_applies(int batch, int seq_len, int head_size) {
     return batch >= kPT || (batch > 1 && !attention_row_fits(seq_len, head_size));
 }
-// Of those, the ones that run on it: it needs enough (head, 64-row tile)
-// workgroups to fill the chip, since each walks its positions serially, while
-// k_attention re-reads K and V once per 4 rows.  They meet at heads x tokens x
-// head size of about 2^20.  Whole prompts, tiled against k_attention: 1B shape
-// (32 heads of 64) 128 tokens 4.90 / 1.92 ms, 512 5.36 / 4.77, 700 6.91 /
-// 6.86, 1000 8.62 / 10.1; SmolLM2 (9 heads of 64) 512 tokens 5.44 / 2.52,
-// 1400 10.4 / 7.86, 2000 14.5 / 12.9.  64 tokens onto 1200, 32 heads of 64:
-// 242 / 48.8 us.
+// Of those, the ones that run on it.  Its time is that of one (head, 64-row
+// tile) workgroup walking the positions serially, until the workgroups fill
+// the chip; k_attention's grows with the rows' work, heads x tokens x head
+// size (both with the context).  They meet at the units below (of 2^18), by
+// how many 4-row workgroups k_attention's score rows leave a CU: three (up to
+// 52 KiB each), two, or none (two rows per workgroup).  Measured, tiled /
+// k_attention us, at units u:
+//   head size 64,  three:  u 4.4 347 / 275, 4.4 (1200 on) 276 / 233,
+//                          5.5 (2000 on) 577 / 597, 8 204 / 206
+//   head size 128, three:  u 6.2 238 / 152, 8 (1200 on) 524 / 540
+//   head size 32,  three:  u 2.7 165 / 99, 3.9 (2000 on) 613 / 612, 5.8 235 / 250
+//   head size 64,  two:    u 2 (2600 on) 573 / 367, 3.1 630 / 592, 4 602 / 650
+//   head size 128, two:    u 4 (2600 on) 622 / 475-555, 6.2 840 / 974
+//   head size 32,  two:    u 2 (2600 on) 562 / 450, 2.7 643 / 630
+//   two-row workgroups:    u 2 .68 to .83 of the tiled time, 2.9 .86 to 1.4
 bool prompt_attn_tiled(int batch, int seq_len, int n_heads, int head_size) {
     if (!prompt_attn_applies(batch, seq_len, head_size)) return false;
     if (head_size != 32 && head_size != 64 && head_size != 128) return true;   // (refused there)
-    return attention_rows_fit(seq_len, head_size) < 4 || (long)batch * n_heads * head_size > (1l << 20);
+    constexpr int kThree[3] = {3, 5, 6}, kTwo[3] = {2, 3, 4};   // head sizes 32, 64, 128
+    const int hs = head_size == 32 ? 0 : (head_size == 64 ? 1 : 2);
+    const int fit = attention_rows_fit(seq_len, head_size);
+    const int units = fit == 4   ? (attention_rows4_three_per_cu(seq_len, head_size) ? kThree[hs] : kTwo[hs])
+                      : fit == 2 ? 2
+                                 : 0;
+    return (long)batch * n_heads * head_size > (long)units << 18;
 }
 
 // ---------------------------------------------------------------------------
