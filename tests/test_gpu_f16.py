@@ -39,9 +39,11 @@ def _pair(oracle, model_dir, name):
 
 
 # one case per tile of the batched kernel (by its number of outputs), with
-# partial row, token and column tiles, and both sides of the first bound
+# partial row, token and column tiles, and both sides of the first bound; past
+# 3 M outputs the 2x4 chains (7001 x 433) and the 64 x 64 tiles (16381 x 190
+# and 16321 x 189: one and several column tiles, partial row and token tiles)
 @pytest.mark.parametrize("o,n,batch", [(33, 32, 2), (17, 96, 17), (6400, 32, 16), (6401, 32, 16), (3001, 160, 33),
-                                       (8191, 64, 90), (7001, 96, 433)])
+                                       (8191, 64, 90), (7001, 96, 433), (16381, 32, 190), (16321, 160, 189)])
 def test_matmul_f32_batch_tiles(gpu, oracle, o, n, batch):
     from yallma3_mini_inference_amd.weight_type import QuantizedWeight, matmul_f32
     rng = np.random.default_rng(o + n + batch)

@@ -13,9 +13,8 @@
 //   each, fed from LDS by three product wavefronts (below).  The prologue
 //   can apply RMSNorm (util.rs:389-426) to the input row, and the epilogue
 //   add the residual or form SwiGLU from gate/up row pairs;
-//   batches: a workgroup takes 64 rows x 64 tokens, each lane running 16
-//   token chains of its row, the weight and activation tiles shared through
-//   LDS.
+//   batches: each lane runs 1 to 16 chains, the weight and activation tiles
+//   of its workgroup (32 x 16 to 64 x 64 outputs) shared through LDS.
 #include <hip/hip_runtime.h>
 
 #include "yl_blocks.h"
@@ -362,7 +361,7 @@ __global__ void k_swiglu_pairs(const float* __restrict__ raw, int hidden, float*
 // Bound: two f32 operations per product (the product and the sum are rounded
 // apart) plus one widening per RR = 1 row and column, and, while the chip is
 // not full, the chain of n dependent sums.  So few outputs take one chain
-// per lane and many take 4 x 4, which read each LDS word for 4 products.
+// per lane and many take 2 x 4, which read each LDS word for 2 or 4 products.
 constexpr int kFbKT = 64;            // columns per tile (32: 3 to 10% slower)
 
 template <int RR, int CC, int TL, int WT>
@@ -491,6 +490,103 @@ __global__ __launch_bounds__(256) void k_matmul_f16_batch(const uint16_t* __rest
         }
 }
 
+// Many outputs.  A workgroup owns 64 rows x 64 tokens: lane r of wavefront w
+// runs the chains of row r for the 16 tokens 16w .. 16w+15, one accumulator
+// each, so one widened weight serves 16 products and every LDS read of
+// activations is a broadcast.  Per K tile of 32 columns the weights ([64
+// rows][32 halves], row stride 80 bytes) and the activations ([32 columns]
+// [64 tokens] f32, read as vf4 of 4 tokens) sit in LDS, double-buffered, as
+// in k_matmul_f16_batch.  Bound: the two f32 operations per product, with
+// the chip full.
+constexpr int kFwRows = 64;          // rows per workgroup (lane = row)
+constexpr int kFwTok = 64;           // tokens per workgroup (16 per wavefront)
+constexpr int kFwKT = 32;            // columns per tile
+constexpr int kFwWStride = 40;       // halves per weight row in LDS (32 + 8: 16-byte aligned, spread banks)
+constexpr int kFwXStride = kFwTok + 4;   // floats per activation column in LDS
+
+template <int EPI>
+__global__ __launch_bounds__(256) void k_matmul_f16_wide(const uint16_t* __restrict__ w, int n, int o,
+                                                          const float* __restrict__ x, int batch,
+                                                          float* __restrict__ out, int out_ld) {
+    __shared__ __align__(16) uint16_t wt[2][kFwRows * kFwWStride];
+    __shared__ __align__(16) float xt[2][kFwKT * kFwXStride];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int row0 = blockIdx.x * kFwRows, tok0 = blockIdx.y * kFwTok;
+    const int ntile = (n + kFwKT - 1) / kFwKT;
+    // loader thread i: weight chunk (row i / 4, halves 8 (i % 4) .. +8) and two
+    // activation float4
+    const int wr_row = tid >> 2, wr_c = (tid & 3) * 8;
+    uint4 wreg;
+    vf4 xreg[2];
+    auto load = [&](int t) {
+        const int k0 = t * kFwKT;
+        const int r = min(row0 + wr_row, o - 1);
+        wreg = *reinterpret_cast<const uint4*>(w + (size_t)r * n + min(k0 + wr_c, n - 8));
+        // activations: 64 tokens x 32 columns = 512 float4; thread i takes
+        // float4 i and i + 256: token (j / 8), columns 4 (j % 8) .. +3
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int j = tid + 256 * h;
+            const int tk = min(tok0 + (j >> 3), batch - 1);
+            xreg[h] = *reinterpret_cast<const vf4*>(x + (size_t)tk * n + min(k0 + 4 * (j & 7), n - 4));
+        }
+    };
+    auto store = [&](int b) {
+        *reinterpret_cast<uint4*>(&wt[b][wr_row * kFwWStride + wr_c]) = wreg;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int j = tid + 256 * h;
+            const int tk = j >> 3, c = 4 * (j & 7);
+            xt[b][(c + 0) * kFwXStride + tk] = xreg[h].x;
+            xt[b][(c + 1) * kFwXStride + tk] = xreg[h].y;
+            xt[b][(c + 2) * kFwXStride + tk] = xreg[h].z;
+            xt[b][(c + 3) * kFwXStride + tk] = xreg[h].w;
+        }
+    };
+    load(0);
+    store(0);
+    __syncthreads();
+    float acc[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
+    for (int t = 0; t < ntile; t++) {
+        const int b = t & 1;
+        if (t + 1 < ntile) load(t + 1);
+        const int kn = min(kFwKT, n - t * kFwKT);   // 32 (n % 32 == 0)
+        const uint16_t* wrow = &wt[b][lane * kFwWStride];
+        const float* xc = &xt[b][16 * wave];
+#pragma unroll
+        for (int c8 = 0; c8 < kFwKT / 8; c8++) {
+            if (8 * c8 >= kn) break;
+            float wf[8];
+            widen8(*reinterpret_cast<const uint4*>(wrow + 8 * c8), wf);
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) {
+                const float* xk = xc + (8 * c8 + kk) * kFwXStride;
+                const vf4 x0 = *reinterpret_cast<const vf4*>(xk), x1 = *reinterpret_cast<const vf4*>(xk + 4),
+                          x2 = *reinterpret_cast<const vf4*>(xk + 8), x3 = *reinterpret_cast<const vf4*>(xk + 12);
+                const float xs[16] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w,
+                                      x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[i] = fadd(acc[i], fmul(xs[i], wf[kk]));
+            }
+        }
+        if (t + 1 < ntile) store(b ^ 1);
+        __syncthreads();
+    }
+    const int row = row0 + lane;
+    if (row < o) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int tk = tok0 + 16 * wave + i;
+            if (tk < batch) {
+                float* dst = out + (size_t)tk * out_ld + row;
+                *dst = EPI == 0 ? acc[i] : fadd(*dst, acc[i]);
+            }
+        }
+    }
+}
+
 // ------------------------------------------------------------------ QKV
 // raw [batch][att + 2 kv] (q | k | v rows of the fused projection) ->
 // RoPE on q and k (util.rs:653-718 pairs (2i, 2i+1) of each head; util.rs
@@ -547,19 +643,34 @@ hipError_t launch_matmul_f16(const uint16_t* w, int n, int o, const float* x, in
                              int epi, hipStream_t s) {
     if (n % 32 || n <= 0 || o <= 0 || batch <= 0 || epi < 0 || epi > 1) return hipErrorInvalidValue;
     if (batch == 1) return launch_f16_gemv(w, n, o, x, nullptr, 0.0f, epi, out, s);
+    // Measured (us; rows x columns, tokens; 64 x 64: k_matmul_f16_wide):
+    //                      1x1     1x2     1x4     2x4    64 x 64
+    //   2048 x 2048, 8     24.9    34.4    52      88      205
+    //   2048 x 2048, 48    29.4    35.3    53.9    87      205
+    //   2048 x 2048, 190   65      57      70      91      206
+    //   3072 x 2048, 300   138     120     112     113     207
+    //   2048 x 8192, 512   562     459     428     442     820
+    //   8000 x 2048, 512   538     437     401     372     355
+    //   8000 x 2048, 700                           499     524
+    //   16384 x 2048, 190                          287     279
+    //   16384 x 2048, 512                          716     666
+    //   28672 x 4096, 190                          993     1042
+    //   28672 x 4096, 300                          1599    1485
+    // Past 3 M outputs a CU takes 5% less per output with 64 x 64 tiles, and
+    // the 32 x 64 tiles of 2x4 win where they end in a less empty last round.
     const long outs = (long)o * batch;
-    // Measured (us; 64 rows x 64 tokens per workgroup, 16 chains per lane
-    // before; rows x columns, tokens):
-    //                     1x1     1x2     1x4     2x4    before
-    //   2048 x 2048, 8    24.9    34.4    52      88      205
-    //   2048 x 2048, 48   29.4    35.3    53.9    87      205
-    //   2048 x 2048, 190  65      57      70      91      206
-    //   3072 x 2048, 300  138     120     112     113     207
-    //   2048 x 8192, 512  562     459     428     442     820
-    //   8000 x 2048, 512  538     437     401     372     373
     if (outs <= 102400) return launch_fb<1, 1, 8, 2>(w, n, o, x, batch, out, out_ld, epi, s);
     if (outs <= 512000) return launch_fb<1, 2, 8, 2>(w, n, o, x, batch, out, out_ld, epi, s);
     if (outs <= 3000000) return launch_fb<1, 4, 4, 2>(w, n, o, x, batch, out, out_ld, epi, s);
+    const auto per_cu = [&](int rows, int toks) {   // workgroups of the busiest of 256 CUs
+        return ((long)((o + rows - 1) / rows) * ((batch + toks - 1) / toks) + 255) / 256;
+    };
+    if (19 * per_cu(kFwRows, kFwTok) <= 10 * per_cu(32, 64)) {
+        auto k = epi == 0 ? k_matmul_f16_wide<0> : k_matmul_f16_wide<1>;
+        hipLaunchKernelGGL(k, dim3((o + kFwRows - 1) / kFwRows, (batch + kFwTok - 1) / kFwTok), dim3(256), 0, s, w, n, o,
+                           x, batch, out, out_ld);
+        return hipGetLastError();
+    }
     return launch_fb<2, 4, 4, 4>(w, n, o, x, batch, out, out_ld, epi, s);
 }
 
