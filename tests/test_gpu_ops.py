@@ -197,6 +197,16 @@ def test_matmul_mfma_tiles(gpu, oracle, fmt, batch, n, o):
     assert_bits(out, ref)
 
 
+# the last Q8_0 call of 4 to 15 tokens on the GEMV and the first on the GEMM, by
+# rows and blocks: up to 64 blocks (up to 4096 rows, more), rows of one
+# wavefront each, up to 128 blocks, more
+@pytest.mark.parametrize("batch,n,o", [(9, 2048, 3666), (9, 2048, 3667), (4, 288, 7499), (4, 288, 7500),
+                                       (10, 4096, 1999), (10, 4096, 2000), (5, 2080, 4999), (5, 2080, 5000),
+                                       (10, 4160, 2049), (11, 4160, 2049)])
+def test_matmul_around_gemv_bound(gpu, oracle, batch, n, o):
+    test_matmul_mfma_tiles(gpu, oracle, 0, batch, n, o)
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("negz", [False, True])
 @pytest.mark.parametrize("batch,n,o", [(96, 512, 384), (2048, 256, 2304)])

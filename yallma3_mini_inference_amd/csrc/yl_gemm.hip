@@ -786,13 +786,32 @@ bool gemm_supported(const GemvArgs& a, int wfmt, int epi, int M) {
 }
 
 // The GEMV's time grows with tokens x rows x blocks (about 4 ps per token and
-// row-block in Q8_0, 1.7 ps in Q4_0), the GEMM's below a full chip only with
-// the chain, about 0.1 us per block: they meet at tokens x rows of 20,000
-// (Q8_0) and 56,000 (Q4_0).  Measured, GEMV against GEMM: 8192 x 2048 Q8_0
-// at 4 tokens 12.2 / 10.1 us, at 8 20.3 / 10.2; 2048 x 8192 Q8_0 at 8 tokens
-// 25.3 / 25.3, at 12 35.7 / 25.4; 4096 x 4096 Q4_0 at 12 14.6 / 16.7.
-bool gemm_preferred(int wfmt, int o, int M) {
-    return M >= 16 || (M >= 4 && (long)M * o >= (wfmt == kQ4 ? 56000 : 20000));
+// row-block in Q8_0, 1.7 ps in Q4_0; less while its rows do not fill the chip,
+// up to 64 blocks or 4096 rows, and more with one wavefront per row, up to
+// 2048 rows of 128 blocks and more), the GEMM's below a full chip only with
+// the chain, about 0.1 us per block.  They meet at the tokens x rows below.
+// Measured, us, GEMV / GEMM (rows x columns Q8_0 unless named, tokens):
+//   2048 x 2048, 15    7.2 / 8.7      8192 x 2048, 4     12.2 / 10.1
+//   4096 x 2048, 8     8.8 / 9.3      6144 x 2048, 5     10.1 / 9.1
+//   3072 x 2048, 12    9.0 / 8.8      3072 x 4096, 8     12.0 / 14.3
+//   4096 x 4096, 6     16.3 / 14.0    6144 x 4096, 4     14.0 / 14.6
+//   2048 x 8192, 8     23.4 / 24.1    2048 x 8192, 12    33.3 / 24.1
+//   4096 x 8192, 5     24.2 / 25.0    4096 x 8192, 6     29.8 / 25.0
+//   Q4_0 4096 x 4096, 12   13.6 / 15.5   Q4_0 6144 x 4096, 12   20.2 / 16.0
+// With a normalization (`norm`: the QKV and gate/up rows of a model) the GEMV
+// normalizes in every workgroup and the GEMM behind a kernel of its own.
+// Whole prompts, us, GEMV / GEMM: four layers of the 1B shape, QKV at 14
+// tokens 455 / 364; six of dim 1024, gate/up at 8 tokens 363 / 328; SmolLM2,
+// gate/up at 8 tokens 1202 / 1258.
+bool gemm_preferred(int wfmt, int o, int nb, int M, bool norm) {
+    if (M >= 16 || M < 4) return M >= 16;
+    long bound;
+    if (norm) bound = wfmt == kQ4 ? 112000 : 40000;
+    else if (wfmt == kQ4) bound = 56000;
+    else if (nb <= 64) bound = o <= 4096 ? 33000 : 30000;
+    else if (nb >= 128 && o <= 2048) bound = 20000;
+    else bound = nb <= 128 ? 25000 : 22000;
+    return (long)M * o >= bound;
 }
 
 hipError_t launch_gemm(const GemvArgs& a, int wfmt, int epi, int M, hipStream_t st) {

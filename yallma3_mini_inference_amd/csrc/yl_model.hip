@@ -884,7 +884,10 @@ enum OpClass : int { kOpQkv = 0, kOpAttn = 1, kOpWo = 2, kOpW13 = 3, kOpW2 = 4, 
 // Prompt batches from this many tokens may run their projections on the int8
 // MFMA GEMM (activations normalized and quantized once per row first) where
 // gemm_preferred says so; the f32-scaled Q8 models, whose other path is the
-// tile kernel, always do from kGemmMinTokensQ8g on.
+// tile kernel, always do from kGemmMinTokensQ8g on: prompts of 4 / 8 / 15
+// tokens through four layers of the 1B shape, tile kernel against GEMM, us,
+// group size 32 731 / 895 / 1335 against 412 / 413 / 420, 64 734 / 798 / 1057
+// against 390 / 392 / 395, 128 779 / 791 / 1143 against 386 / 386 / 390.
 constexpr int kGemmMinTokens = 8;
 constexpr int kGemmMinTokensQ8g = 4;
 
@@ -923,11 +926,8 @@ hipError_t enqueue_op_gemm(const yl_model* m, yl_session* s, int cls, int l, int
         return hipErrorNotSupported;
     }
     a.qs = w->qs; a.d = w->d; a.n = w->n; a.o = w->o; a.nb = w->nb;
-    // (the GEMV normalizes in its prologue, the GEMM behind a kernel of its
-    // own: half the rows count.  SmolLM2's 3072 gate/up rows at 8 tokens: a
-    // prompt of 1258 us with the GEMM, 1202 without)
     const bool norm = cls == kOpQkv || cls == kOpW13;
-    if (!gemm_supported(a, w->fmt, epi, batch) || !gemm_preferred(w->fmt, norm ? w->o / 2 : w->o, batch))
+    if (!gemm_supported(a, w->fmt, epi, batch) || !gemm_preferred(w->fmt, w->o, w->nb, batch, norm))
         return hipErrorNotSupported;
     hipError_t e = hipSuccess;
     if (prologue && norm) {
@@ -1546,7 +1546,7 @@ yl_status yl_matmul(float* out, yl_format fmt, const int8_t* xq, const float* xs
     GemvArgs a{};
     a.qs = w->m.qs; a.d = w->m.d; a.n = w->m.n; a.o = w->m.o; a.nb = w->m.nb;
     a.xq = xq; a.xs = xs; a.out = out; a.accumulate_cols = (int)(o / 4 * 4);
-    const bool mfma = gemm_preferred(w->m.fmt, (int)o, (int)batch) && gemm_supported(a, w->m.fmt, kEpiStore, (int)batch);
+    const bool mfma = gemm_preferred(w->m.fmt, (int)o, w->m.nb, (int)batch) && gemm_supported(a, w->m.fmt, kEpiStore, (int)batch);
     const hipError_t e = mfma ? launch_gemm(a, w->m.fmt, kEpiStore, (int)batch, (hipStream_t)stream)
                               : launch_gemv(a, w->m.fmt, kEpiStore, (int)batch, (hipStream_t)stream);
     return e == hipSuccess ? YL_OK : hip_fail(e, "matmul launch");
@@ -1577,7 +1577,7 @@ yl_status yl_matmul_bench(const yl_weight* const* ws, size_t count, const int8_t
         GemvArgs a{};
         a.qs = w.qs; a.d = w.d; a.n = w.n; a.o = w.o; a.nb = w.nb;
         a.xq = xq; a.xs = xs; a.out = out; a.accumulate_cols = 0;
-        const bool mfma = gemm_preferred(w.fmt, w.o, (int)batch) && gemm_supported(a, w.fmt, kEpiStore, (int)batch);
+        const bool mfma = gemm_preferred(w.fmt, w.o, w.nb, (int)batch) && gemm_supported(a, w.fmt, kEpiStore, (int)batch);
         ec = mfma ? launch_gemm(a, w.fmt, kEpiStore, (int)batch, st) : launch_gemv(a, w.fmt, kEpiStore, (int)batch, st);
     }
     if (e == hipSuccess) e = hipStreamEndCapture(st, &g);
