@@ -510,6 +510,15 @@ def test_row_kernel_edges(gpu, oracle, size, batch, qfmt):
             assert_bits(got[1], os_)
 
 
+# rows of one to four wavefronts per workgroup, full and partial, and SwiGLU
+# rows split evenly over two and three workgroups
+@pytest.mark.parametrize("size,batch,qfmt", [(512, 2, 0), (544, 3, 1), (576, 5, 0), (1024, 2, 1), (1056, 2, 0), (1536, 3, 1),
+                                             (2016, 2, 0), (2336, 2, 1)])
+def test_row_kernel_widths(gpu, oracle, size, batch, qfmt):
+    test_row_kernel_edges(gpu, oracle, size, batch, qfmt)
+    test_row_kernel_edges(gpu, oracle, size, batch, -1)
+
+
 def test_serial_sum_exact(gpu):
     # the softmax denominator's serial sum by one wavefront (forward.rs:356-361)
     import sys, os
