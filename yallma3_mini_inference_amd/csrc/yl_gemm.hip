@@ -551,8 +551,9 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
     }
     };
 
-    // (small tiles read the residual ahead of the K loop, off the tail)
-    constexpr bool kResidEarly = EPI == kEpiResid && WM * WN * R <= 16;
+    // (16 x 16 tiles read the residual ahead of the K loop, off the tail; the
+    // 16 registers of a 32 x 32 tile's spilled there, 5 to 12 of them)
+    constexpr bool kResidEarly = EPI == kEpiResid && R == 4;
     [[maybe_unused]] float resid[WM][WN][R];
     if constexpr (kResidEarly) {
 #pragma unroll
