@@ -14,8 +14,8 @@
 // (the convert folded away; see `bias` in k_gemm), one product and one sum;
 // with f32 scales a convert, two products and one sum.
 //
-// Tile: a workgroup of GM x GN wavefronts; each wavefront owns WM x WN MFMA
-// tiles of T tokens x T weight rows.  MFMA lane layout (gfx950), g = l / T:
+// Tile: a workgroup of GM x GN wavefronts; each wavefront owns one MFMA tile
+// of T tokens x T weight rows.  MFMA lane layout (gfx950), g = l / T:
 // operand lane l holds row l%T (token for A, weight row for B) and, of the
 // block's 32 bytes, 8*g .. +7 (T = 16) or 16*g .. +15 (T = 32); result
 // register i of lane l is (token 4*g + i (T = 16) or (i%4) + 8*(i/4) + 4*g
@@ -39,8 +39,6 @@
 // activations are quantized in the same groups.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "yl_blocks.h"
 #include "yl_device.h"
 #include "yl_internal.h"
@@ -54,14 +52,14 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 template <int WF>
 constexpr int gm_bpg() { return WF == kQ8S64 ? 2 : (WF == kQ8S128 ? 4 : 1); }
 
-// One tile configuration: T x T MFMA tiles, WM x WN of them per wavefront,
-// GM x GN wavefronts, KB blocks per stage, NST stages, registers for OCC
-// wavefronts per SIMD; DEEP: a stage's operands read ahead (see k_gemm).
-template <int T_, int WM_, int WN_, int GM_, int GN_, int KB_, int NST_, int OCC_, bool DEEP_ = false>
+// One tile configuration: T x T MFMA tiles, one per wavefront, GM x GN
+// wavefronts, KB blocks per stage, NST stages, registers for OCC wavefronts
+// per SIMD; DEEP: a stage's operands read ahead (see k_gemm).
+template <int T_, int GM_, int GN_, int KB_, int NST_, int OCC_, bool DEEP_ = false>
 struct GmCfg {
     static constexpr bool DEEP = DEEP_;
-    static constexpr int T = T_, WM = WM_, WN = WN_, GM = GM_, GN = GN_, KB = KB_, NST = NST_, OCC = OCC_;
-    static constexpr int NW = GM * GN, TM = T * WM * GM, TN = T * WN * GN;
+    static constexpr int T = T_, GM = GM_, GN = GN_, KB = KB_, NST = NST_, OCC = OCC_;
+    static constexpr int NW = GM * GN, TM = T * GM, TN = T * GN;
 };
 
 // What one stage holds in LDS, and the DMA instructions that fill it.
@@ -100,11 +98,10 @@ __device__ __forceinline__ int gm_unit(int row, int p) { return row * U + (p ^ (
 // younger stages (D instructions each) are still in flight
 template <int D, int NST>
 __device__ __forceinline__ void gm_wait(int later) {
-    static_assert(NST >= 2 && NST <= 5, "waits below");
+    static_assert(NST >= 2 && NST <= 4, "waits below");
     if (later <= 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     else if (NST == 3 || later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D) : "memory");
-    else if (NST == 4 || later == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NST >= 4 ? 2 * D : 0) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NST >= 5 ? 3 * D : 0) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NST >= 4 ? 2 * D : 0) : "memory");
 }
 
 // 4 Q4_0 bytes (8 nibbles, byte j = elements 2j | 2j+1 << 4) -> 8 int8 in
@@ -153,17 +150,16 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
     // needs just the launch stub)
 #if defined(__HIP_DEVICE_COMPILE__)
     using S = GmStage<WF, C>;
-    constexpr int T = C::T, WM = C::WM, WN = C::WN, KB = C::KB, G = S::G, NW = C::NW;
+    constexpr int T = C::T, KB = C::KB, G = S::G, NW = C::NW;
     constexpr int R = T * T / 64;   // result registers per tile
     constexpr bool kDeep = C::DEEP;
-    static_assert(!kDeep || WM * WN == 1, "one tile per wavefront");
     using MF = GmMfma<T>;
     extern __shared__ __align__(16) unsigned char gsm[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rt = lane % T, lg = lane / T;
     const int wm = wave % C::GM, wn = wave / C::GM;
     const int c0 = blockIdx.x * C::TN, t0 = blockIdx.y * C::TM;
-    const int tw = t0 + T * WM * wm, cw = c0 + T * WN * wn;   // this wavefront's first token and row
+    const int tw = t0 + T * wm, cw = c0 + T * wn;   // this wavefront's first token and row
     const int nst = (a.nb + KB - 1) / KB;
 
     // ---- DMA plan: each instruction's lane offset, once ----
@@ -231,24 +227,21 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         }
     };
 
-    // accumulators: acc[tm][tn][i] = (token tw + T*tm + 4lg + tok_of(i), row cw + T*tn + rt)
-    float acc[WM][WN][R];
+    // accumulators: acc[i] = (token tw + 4lg + tok_of(i), row cw + rt)
+    float acc[R];
     // token offset of register i in a tile, beyond the lane group's 4 * lg
     auto tok_of = [](int i) { return T == 16 ? i : (i & 3) + 8 * (i >> 2); };
     int pos = 0;
     if constexpr (EPI == kEpiQkvRope) pos = a.state->pos;
-    // QKV rows: each lane's stored column within q or k (RoPE pair order)
-    // and its pair index, for its 16-row tiles
-    [[maybe_unused]] int kcol[WN] = {}, qkcol[WN] = {}, qpair[WN] = {};
+    // QKV rows: the lane's stored column within q or k (RoPE pair order) and
+    // its pair index
+    [[maybe_unused]] int kcol = 0, qkcol = 0, qpair = 0;
     if constexpr (EPI == kEpiQkvRope) {
-#pragma unroll
-        for (int tn = 0; tn < WN; tn++) {
-            const int c = cw + T * tn + rt, att = a.att_dim;
-            const int scol = c < att ? c : c - att;   // stored row within q or k
-            kcol[tn] = qk_column(c - att, a.head_size, a.hf_rows);
-            qkcol[tn] = qk_column(scol, a.head_size, a.hf_rows);
-            qpair[tn] = (scol % a.head_size) >> 1;
-        }
+        const int c = cw + rt, att = a.att_dim;
+        const int scol = c < att ? c : c - att;   // stored row within q or k
+        kcol = qk_column(c - att, a.head_size, a.hf_rows);
+        qkcol = qk_column(scol, a.head_size, a.hf_rows);
+        qpair = (scol % a.head_size) >> 1;
     }
     // (lane coordinates opaque per use: the initial values' and the epilogue's
     // addresses are then computed where they are used, not kept across the K
@@ -258,35 +251,29 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         return v;
     };
     auto init_acc = [&]() {
-    const int tl = opaque(tw + 4 * lg), cl = opaque(cw + rt);
+        const int tl = opaque(tw + 4 * lg), c = opaque(cw + rt);
 #pragma unroll
-    for (int tm = 0; tm < WM; tm++)
-#pragma unroll
-        for (int tn = 0; tn < WN; tn++)
-#pragma unroll
-            for (int i = 0; i < R; i++) {
-                float v = 0.0f;
-                const int t = tl + T * tm + tok_of(i);
-                const int c = cl + T * tn;
-                if constexpr (EPI == kEpiStore) {
-                    if (t < M && c < a.o && c < a.accumulate_cols) v = a.out[(size_t)t * a.o + c];
-                } else if constexpr (EPI == kEpiQkvRope) {
-                    // K/V rows accumulate into the cache (forward.rs:166-169);
-                    // q rows start at 0.  A 16-row tile is all q, all k or
-                    // all v (att_dim and kv_dim are multiples of 32), so the
-                    // branches are uniform; token t0 stands in for the rows
-                    // past M in the (then unused) loads.
-                    const int cb = cw + T * tn, att = a.att_dim, kv = a.kv_dim;
-                    if (cb >= att && cb < a.o) {
-                        const int tc = t < M ? t : t0;
-                        const float u = cb < att + kv
-                                            ? a.k_cache[(size_t)kcol[tn] * a.kv_ld + pos + tc]
-                                            : a.v_cache[(size_t)(pos + tc) * kv + (c - att - kv)];
-                        if (t < M) v = u;
-                    }
+        for (int i = 0; i < R; i++) {
+            float v = 0.0f;
+            const int t = tl + tok_of(i);
+            if constexpr (EPI == kEpiStore) {
+                if (t < M && c < a.o && c < a.accumulate_cols) v = a.out[(size_t)t * a.o + c];
+            } else if constexpr (EPI == kEpiQkvRope) {
+                // K/V rows accumulate into the cache (forward.rs:166-169);
+                // q rows start at 0.  A tile's rows are all q, all k or all
+                // v (att_dim and kv_dim are multiples of 32), so the branches
+                // are uniform; token t0 stands in for the rows past M in the
+                // (then unused) loads.
+                const int att = a.att_dim, kv = a.kv_dim;
+                if (cw >= att && cw < a.o) {
+                    const int tc = t < M ? t : t0;
+                    const float u = cw < att + kv ? a.k_cache[(size_t)kcol * a.kv_ld + pos + tc]
+                                                  : a.v_cache[(size_t)(pos + tc) * kv + (c - att - kv)];
+                    if (t < M) v = u;
                 }
-                acc[tm][tn][i] = v;
             }
+            acc[i] = v;
+        }
     };
 
     // f16 block scales (Q8_0, Q4_0): every block dot starts from the int32
@@ -321,67 +308,54 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
     int neg_zero = 0;   // this lane saw a -0 initial value
 
     // lane offsets of the operand reads within a stage
-    const int offA = T * WM * wm * S::UA * 16, offB = S::A + T * WN * wn * S::UB * 16;
+    const int offA = T * wm * S::UA * 16, offB = S::A + T * wn * S::UB * 16;
     const int wsh = (((int)rt & a.nb & 1)) << 4;   // an odd nb: odd rows' scales start in the high half
 
     // the K loop: FUSED.value selects the biased form above
     auto run = [&](auto FUSED) {
     constexpr bool kFused = decltype(FUSED)::value;
-    [[maybe_unused]] typename MF::res gd[WM][WN];   // group dots (G > 1)
+    typename MF::res gd;   // group dot (or the block's, G = 1)
 
-    // one block's operands: both int8 tiles' rows, the activation scales of
-    // the lane's tokens (with a group's last block) and the raw weight scales
+    // one block's operands: both int8 rows, the activation scales of the
+    // lane's tokens (with a group's last block) and the raw weight scale
     struct Ops {
-        typename MF::op av[WM], bv[WN];
-        vf4 xv[WM][R / 4];
-        uint32_t ws[WN];
+        typename MF::op av, bv;
+        vf4 xv[R / 4];
+        uint32_t ws;
     };
     // byte offset of this lane's share of block blk in row rt of a tile
     auto lane_off = [&](int blk) {
         return T == 16 ? gm_unit<S::UA>(rt, 2 * blk + (lg >> 1)) * 16 + 8 * (lg & 1) : gm_unit<S::UA>(rt, 2 * blk + lg) * 16;
     };
-    auto load_ops = [&](const unsigned char* buf, int blk, const uint32_t (&w)[WN], Ops& o) {
-#pragma unroll
-        for (int tm = 0; tm < WM; tm++)
-            o.av[tm] = *reinterpret_cast<const typename MF::op*>(buf + offA + T * tm * S::UA * 16 + lane_off(blk));
-#pragma unroll
-        for (int tn = 0; tn < WN; tn++) {
-            const unsigned char* bt = buf + offB + T * tn * S::UB * 16;
-            if constexpr (WF != kQ4) {
-                o.bv[tn] = *reinterpret_cast<const typename MF::op*>(bt + lane_off(blk));
-            } else if constexpr (T == 16) {   // (the nibbles; unpacked by block())
-                o.bv[tn] = *reinterpret_cast<const uint32_t*>(bt + gm_unit<S::UB>(rt, blk) * 16 + 4 * lg);
-            } else {
-                const uint2 u = *reinterpret_cast<const uint2*>(bt + gm_unit<S::UB>(rt, blk) * 16 + 8 * lg);
-                o.bv[tn] = v4i{(int)u.x, (int)u.y, 0, 0};
-            }
+    auto load_ops = [&](const unsigned char* buf, int blk, uint32_t w, Ops& o) {
+        o.av = *reinterpret_cast<const typename MF::op*>(buf + offA + lane_off(blk));
+        const unsigned char* bt = buf + offB;
+        if constexpr (WF != kQ4) {
+            o.bv = *reinterpret_cast<const typename MF::op*>(bt + lane_off(blk));
+        } else if constexpr (T == 16) {   // (the nibbles; unpacked by block())
+            o.bv = *reinterpret_cast<const uint32_t*>(bt + gm_unit<S::UB>(rt, blk) * 16 + 4 * lg);
+        } else {
+            const uint2 u = *reinterpret_cast<const uint2*>(bt + gm_unit<S::UB>(rt, blk) * 16 + 8 * lg);
+            o.bv = v4i{(int)u.x, (int)u.y, 0, 0};
         }
         if (G == 1 || blk % G == G - 1) {
             const float* xl = reinterpret_cast<const float*>(buf + S::A + S::B) + 4 * lg;
 #pragma unroll
-            for (int tm = 0; tm < WM; tm++)
-#pragma unroll
-                for (int i = 0; i < R / 4; i++)
-                    o.xv[tm][i] = *reinterpret_cast<const vf4*>(xl + ((wm * WM + tm) * S::XW + blk / G) * T + 8 * i);
-#pragma unroll
-            for (int tn = 0; tn < WN; tn++) {
-                if constexpr (S::kF32)
-                    o.ws[tn] = reinterpret_cast<const uint32_t*>(buf + S::A + S::B + S::XS)[blk / G * C::TN + T * (wn * WN + tn) + rt];
-                else o.ws[tn] = w[tn];
-            }
+            for (int i = 0; i < R / 4; i++)
+                o.xv[i] = *reinterpret_cast<const vf4*>(xl + (wm * S::XW + blk / G) * T + 8 * i);
+            if constexpr (S::kF32)
+                o.ws = reinterpret_cast<const uint32_t*>(buf + S::A + S::B + S::XS)[blk / G * C::TN + T * wn + rt];
+            else o.ws = w;
         }
     };
     // Q4_0: the nibbles read, to int8
     auto unpack = [&](Ops& o) {
         if constexpr (WF == kQ4) {
-#pragma unroll
-            for (int tn = 0; tn < WN; tn++) {
-                if constexpr (T == 16) {
-                    o.bv[tn] = __builtin_bit_cast(long, q4_unpack8((uint32_t)o.bv[tn]));
-                } else {
-                    const uint2 x = q4_unpack8((uint32_t)o.bv[tn].x), y = q4_unpack8((uint32_t)o.bv[tn].y);
-                    o.bv[tn] = v4i{(int)x.x, (int)x.y, (int)y.x, (int)y.y};
-                }
+            if constexpr (T == 16) {
+                o.bv = __builtin_bit_cast(long, q4_unpack8((uint32_t)o.bv));
+            } else {
+                const uint2 x = q4_unpack8((uint32_t)o.bv.x), y = q4_unpack8((uint32_t)o.bv.y);
+                o.bv = v4i{(int)x.x, (int)x.y, (int)y.x, (int)y.y};
             }
         }
     };
@@ -396,10 +370,10 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
             cb = fmul(-kBiasF, ws);
         }
     };
-    // one tile's terms onto its sums.  The three (four) steps run over the
+    // the tile's terms onto its sums.  The three (four) steps run over the
     // outputs one step at a time, so that no instruction waits on the one
     // before it.
-    auto fold = [&](const typename MF::res& d, float ws, float cb, const vf4 (&xv)[R / 4], float (&sum)[R]) {
+    auto fold = [&](const typename MF::res& d, float ws, float cb, const vf4 (&xv)[R / 4]) {
         float term[R];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -412,37 +386,22 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         for (int i = 0; i < R; i++) term[i] = fmul(term[i], xv[i / 4][i % 4]);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < R; i++) sum[i] = fadd(sum[i], term[i]);
+        for (int i = 0; i < R; i++) acc[i] = fadd(acc[i], term[i]);
         __builtin_amdgcn_sched_barrier(0);
     };
-    // the block's products and terms
-    auto block = [&](int blk, Ops& o) {
-        constexpr int NT = WM * WN;
-        float wsc[WN], cb[WN];
+    // the block's product and terms; `next` (the next block's reads) is
+    // issued while the MFMA runs
+    auto block = [&](int blk, Ops& o, auto next) {
+        float wsc, cb;
         unpack(o);
-#pragma unroll
-        for (int tn = 0; tn < WN; tn++) scale(o.ws[tn], blk, wsc[tn], cb[tn]);
+        scale(o.ws, blk, wsc, cb);
         const typename MF::res zero = {};
-        if constexpr (G > 1) {
-            // this block's dots join the group's (the first block of a
-            // group starts from zero); the term follows the group's last
-#pragma unroll
-            for (int k = 0; k < NT; k++)
-                gd[k / WN][k % WN] = MF::mul(o.av[k / WN], o.bv[k % WN], blk % G == 0 ? zero : gd[k / WN][k % WN]);
-            if (blk % G != G - 1) return;
-#pragma unroll
-            for (int k = 0; k < NT; k++) fold(gd[k / WN][k % WN], wsc[k % WN], cb[k % WN], o.xv[k / WN], acc[k / WN][k % WN]);
-        } else {
-            // tile k+1's MFMA runs while tile k is folded
-            typename MF::res d[2];
-            const typename MF::res start = kFused ? bias : zero;
-            d[0] = MF::mul(o.av[0], o.bv[0], start);
-#pragma unroll
-            for (int k = 0; k < NT; k++) {
-                if (k + 1 < NT) d[(k + 1) & 1] = MF::mul(o.av[(k + 1) / WN], o.bv[(k + 1) % WN], start);
-                fold(d[k & 1], wsc[k % WN], cb[k % WN], o.xv[k / WN], acc[k / WN][k % WN]);
-            }
-        }
+        // (the first block of a group starts from zero, the others' dots join
+        // it; the term follows the group's last)
+        gd = MF::mul(o.av, o.bv, G > 1 && blk % G ? gd : (kFused ? bias : zero));
+        __builtin_amdgcn_sched_barrier(0);
+        next();
+        if (G == 1 || blk % G == G - 1) fold(gd, wsc, cb, o.xv);
     };
 
 #pragma unroll
@@ -452,8 +411,7 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         // (the initial values are older loads than the stages')
         int flag = 0;
 #pragma unroll
-        for (int k = 0; k < WM * WN * R; k++)
-            flag |= __float_as_uint(acc[k / (R * WN)][k / R % WN][k % R]) == 0x80000000u;
+        for (int i = 0; i < R; i++) flag |= __float_as_uint(acc[i]) == 0x80000000u;
         neg_zero = flag;
         asm volatile("" : "+v"(neg_zero));   // decided here: the initial values do not outlive the loop
     }
@@ -468,27 +426,24 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         cur = cur == C::NST - 1 ? 0 : cur + 1;
         return buf;
     };
-    // the stage's f16 weight scales of this lane's rows, two to a word
-    uint32_t wraw[KB / 2][WN];
+    // the stage's f16 weight scales of this lane's row, two to a word
+    uint32_t wraw[KB / 2];
     auto load_scales = [&](const unsigned char* buf) {
         if constexpr (!S::kF32) {
+            const uint32_t* p = reinterpret_cast<const uint32_t*>(buf + S::A + S::B + S::XS) + (T * wn + rt) * S::WW;
+            uint32_t w[S::WW];
 #pragma unroll
-            for (int tn = 0; tn < WN; tn++) {
-                const uint32_t* p = reinterpret_cast<const uint32_t*>(buf + S::A + S::B + S::XS) + (T * (wn * WN + tn) + rt) * S::WW;
-                uint32_t w[S::WW];
+            for (int i = 0; i < S::WW; i++) w[i] = p[i];
 #pragma unroll
-                for (int i = 0; i < S::WW; i++) w[i] = p[i];
-#pragma unroll
-                for (int i = 0; i < KB / 2; i++) wraw[i][tn] = __builtin_amdgcn_alignbit(w[i + 1], w[i], wsh);
-            }
+            for (int i = 0; i < KB / 2; i++) wraw[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], wsh);
         }
     };
     const int full = a.nb / KB;
     if constexpr (kDeep) {
-        // one tile per wavefront: a block's work (12 VALU instructions) is
-        // shorter than the latencies around it, so a whole stage's operands
-        // are read while the previous stage is folded, and its MFMAs issued
-        // back to back ahead of its folds
+        // a 16 x 16 tile's block (12 VALU instructions) is shorter than the
+        // latencies around it, so a whole stage's operands are read while the
+        // previous stage is folded, and its MFMAs issued back to back ahead
+        // of its folds
         Ops q[2][KB];
         auto load_stage = [&](int s, Ops (&o)[KB]) {
             const unsigned char* buf = arrive(s);
@@ -502,14 +457,14 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
             for (int blk = 0; blk < KB; blk++) {
                 unpack(o[blk]);
                 const typename MF::res zero = {};
-                d[blk / G] = MF::mul(o[blk].av[0], o[blk].bv[0], blk % G ? d[blk / G] : kFused ? bias : zero);
+                d[blk / G] = MF::mul(o[blk].av, o[blk].bv, blk % G ? d[blk / G] : kFused ? bias : zero);
             }
             if (s + 1 < full) load_stage(s + 1, nx);
 #pragma unroll
             for (int blk = G - 1; blk < KB; blk += G) {
                 float wsc, cb;
-                scale(o[blk].ws[0], blk, wsc, cb);
-                fold(d[blk / G], wsc, cb, o[blk].xv[0], acc[0][0]);
+                scale(o[blk].ws, blk, wsc, cb);
+                fold(d[blk / G], wsc, cb, o[blk].xv);
             }
         };
         if (full > 0) load_stage(0, q[0]);
@@ -528,8 +483,9 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         load_ops(buf, 0, wraw[0], o[0]);
 #pragma unroll
         for (int blk = 0; blk < KB; blk++) {
-            if (blk + 1 < KB) load_ops(buf, blk + 1, wraw[(blk + 1) / 2], o[(blk + 1) & 1]);
-            block(blk, o[blk & 1]);
+            block(blk, o[blk & 1], [&] {
+                if (blk + 1 < KB) load_ops(buf, blk + 1, wraw[(blk + 1) / 2], o[(blk + 1) & 1]);
+            });
         }
     }
     // the blocks of a last, partial stage
@@ -538,15 +494,11 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         load_scales(buf);
 #pragma unroll 1
         for (int blk = 0; blk < a.nb - full * KB; blk++) {
-            uint32_t w[WN];
-#pragma unroll
-            for (int tn = 0; tn < WN; tn++) {
-                w[tn] = wraw[0][tn];
-                if constexpr (KB > 2) w[tn] = blk >= 2 ? wraw[1][tn] : w[tn];
-            }
+            uint32_t w = wraw[0];
+            if constexpr (KB > 2) w = blk >= 2 ? wraw[1] : w;
             Ops o;
             load_ops(buf, blk, w, o);
-            block(blk, o);
+            block(blk, o, [] {});
         }
     }
     };
@@ -554,12 +506,12 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
     // (16 x 16 tiles read the residual ahead of the K loop, off the tail; the
     // 16 registers of a 32 x 32 tile's spilled there, 5 to 12 of them)
     constexpr bool kResidEarly = EPI == kEpiResid && R == 4;
-    [[maybe_unused]] float resid[WM][WN][R];
+    [[maybe_unused]] float resid[R];
     if constexpr (kResidEarly) {
 #pragma unroll
-        for (int k = 0; k < WM * WN * R; k++) {
-            const int t = min(tw + T * (k / (R * WN)) + 4 * lg + tok_of(k % R), M - 1), c = min(cw + T * (k / R % WN) + rt, a.o - 1);
-            resid[k / (R * WN)][k / R % WN][k % R] = a.x[(size_t)t * a.o + c];
+        for (int i = 0; i < R; i++) {
+            const int t = min(tw + 4 * lg + tok_of(i), M - 1), c = min(cw + rt, a.o - 1);
+            resid[i] = a.x[(size_t)t * a.o + c];
         }
     }
     init_acc();
@@ -567,10 +519,7 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         run(std::true_type{});
         bool flag = neg_zero != 0;
 #pragma unroll
-        for (int k = 0; k < WM * WN * R; k++) {
-            const float v = acc[k / (R * WN)][k / R % WN][k % R];
-            flag = flag || v != v;
-        }
+        for (int i = 0; i < R; i++) flag = flag || acc[i] != acc[i];
         if (flag) redo = 1;
         __syncthreads();   // every flag is in; every wavefront is done with the LDS stages
         if (redo) {
@@ -582,115 +531,73 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
         run(std::false_type{});
     }
 
-    const int tl = opaque(tw + 4 * lg), cl = opaque(cw + rt);
-    // SwiGLU (forward.rs:220-237) of one output of the 64-row group
-    // [32 gate | 32 up], with expf's constants in registers
-    [[maybe_unused]] const ExpfK ek = EPI == kEpiSwiglu ? expf_k_regs() : expf_k_imm();
+    const int tl = opaque(tw + 4 * lg), c = opaque(cw + rt);
     if constexpr (EPI == kEpiSwiglu) {
-        auto swiglu = [&](float g, float u) {
+        // SwiGLU (forward.rs:220-237) of the 64-row groups [32 gate | 32 up],
+        // with expf's constants in registers.  A group's rows are spread over
+        // wavefronts: exchange the sums through LDS (the stages are done),
+        // then one 32-lane half per (token, group)
+        const ExpfK ek = expf_k_regs();
+        static_assert(C::TN % 64 == 0, "whole 64-row groups per workgroup");
+        constexpr int LD = C::TN + 4;
+        float* ex = reinterpret_cast<float*>(gsm);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < R; i++) ex[(tl - t0 + tok_of(i)) * LD + c - c0] = acc[i];
+        __syncthreads();
+        constexpr int NG = C::TN / 64;
+        const int l32 = threadIdx.x & 31;
+        for (int it = threadIdx.x >> 5; it < C::TM * NG; it += 2 * NW) {
+            const int t = t0 + it / NG, q = it % NG, grp = c0 / 64 + q;
+            const bool ok = t < M && c0 + 64 * q < a.o;
+            const float g = ex[(it / NG) * LD + 64 * q + l32], u = ex[(it / NG) * LD + 64 * q + 32 + l32];
             const float den = fadd(1.0f, expf_rn(-g, ek));
-            return fmul(g / den, u);
-        };
-        auto scale_of = [&](float am) { return a.h_fmt == kQ4 ? group_scale<kQ4>(am) : group_scale<kQ8>(am); };
-        auto quant = [&](float h, float sc) { return (int8_t)(a.h_fmt == kQ4 ? quant_one<kQ4>(h, sc) : quant_one<kQ8>(h, sc)); };
-        if constexpr (T == 32 && WN % 2 == 0) {
-            // a wavefront owns whole groups: tile 2q the gate rows, 2q+1 the
-            // up rows; 32 lanes hold one token's group of h
-#pragma unroll
-            for (int tm = 0; tm < WM; tm++)
-#pragma unroll
-                for (int q = 0; q < WN / 2; q++)
-#pragma unroll
-                    for (int i = 0; i < R; i++) {
-                        const int t = tl + T * tm + tok_of(i), grp = cw / 64 + q;
-                        const bool ok = t < M && cw + 64 * q < a.o;
-                        const size_t base = (size_t)t * a.hidden + (size_t)grp * kGroup;
-                        const float h = swiglu(acc[tm][2 * q][i], acc[tm][2 * q + 1][i]);
-                        if (a.h_f32 && ok) a.h_f32[base + rt] = h;
-                        if (!a.hq) continue;   // f32 h only (quantized afterwards in the model's groups)
-                        const float am = fmaxf(group_max(fabsf(h), 32), 0.0f);
-                        const float sc = scale_of(am);
-                        const int8_t qv = quant(h, sc);
-                        if (ok) {
-                            a.hq[base + rt] = qv;
-                            if (rt == 0) a.hs[(size_t)t * (a.hidden / kGroup) + grp] = sc;
-                        }
-                    }
-        } else {
-            // the group's rows are spread over wavefronts: exchange the sums
-            // through LDS (the stages are done), then one 32-lane half per
-            // (token, group)
-            static_assert(EPI != kEpiSwiglu || C::TN % 64 == 0, "whole 64-row groups per workgroup");
-            constexpr int LD = C::TN + 4;
-            float* ex = reinterpret_cast<float*>(gsm);
-            __syncthreads();
-#pragma unroll
-            for (int tm = 0; tm < WM; tm++)
-#pragma unroll
-                for (int tn = 0; tn < WN; tn++)
-#pragma unroll
-                    for (int i = 0; i < R; i++)
-                        ex[(tl - t0 + T * tm + tok_of(i)) * LD + cl - c0 + T * tn] = acc[tm][tn][i];
-            __syncthreads();
-            constexpr int NG = C::TN / 64;
-            const int l32 = threadIdx.x & 31;
-            for (int it = threadIdx.x >> 5; it < C::TM * NG; it += 2 * NW) {
-                const int t = t0 + it / NG, q = it % NG, grp = c0 / 64 + q;
-                const bool ok = t < M && c0 + 64 * q < a.o;
-                const float h = swiglu(ex[(it / NG) * LD + 64 * q + l32], ex[(it / NG) * LD + 64 * q + 32 + l32]);
-                const size_t base = (size_t)t * a.hidden + (size_t)grp * kGroup;
-                if (a.h_f32 && ok) a.h_f32[base + l32] = h;
-                if (!a.hq) continue;
-                const float am = fmaxf(group_max(fabsf(h), 32), 0.0f);
-                const float sc = scale_of(am);
-                const int8_t qv = quant(h, sc);
-                if (ok) {
-                    a.hq[base + l32] = qv;
-                    if (l32 == 0) a.hs[(size_t)t * (a.hidden / kGroup) + grp] = sc;
-                }
+            const float h = fmul(g / den, u);
+            const size_t base = (size_t)t * a.hidden + (size_t)grp * kGroup;
+            if (a.h_f32 && ok) a.h_f32[base + l32] = h;
+            if (!a.hq) continue;   // f32 h only (quantized afterwards in the model's groups)
+            const float am = fmaxf(group_max(fabsf(h), 32), 0.0f);
+            const float sc = a.h_fmt == kQ4 ? group_scale<kQ4>(am) : group_scale<kQ8>(am);
+            const int8_t qv = (int8_t)(a.h_fmt == kQ4 ? quant_one<kQ4>(h, sc) : quant_one<kQ8>(h, sc));
+            if (ok) {
+                a.hq[base + l32] = qv;
+                if (l32 == 0) a.hs[(size_t)t * (a.hidden / kGroup) + grp] = sc;
             }
         }
     } else {
 #pragma unroll
-        for (int tm = 0; tm < WM; tm++)
-#pragma unroll
-            for (int tn = 0; tn < WN; tn++)
-#pragma unroll
-                for (int i = 0; i < R; i++) {
-                    const int t = tl + T * tm + tok_of(i);
-                    const bool tok_ok = t < M;
-                    const int c = cl + T * tn;
-                    const float v = acc[tm][tn][i];
-                    if constexpr (EPI == kEpiQkvRope) {
-                        // rope_gguf (util.rs:653-718) on q and k pairs (2j, 2j+1):
-                        // the pair partner is the neighbouring lane
-                        const float other = dpp_mov<0xB1>(v);
-                        // (uniform branches on the 16-row tile, as in the
-                        // initial values)
-                        const int cb = cw + T * tn;
-                        const int att = a.att_dim, kv = a.kv_dim, hd = a.head_size;
-                        if (cb >= att + kv) {
-                            if (tok_ok && cb < a.o) a.v_cache[(size_t)(pos + t) * kv + (c - att - kv)] = v;
-                        } else {
-                            const int tc = tok_ok ? t : t0;
-                            const float cs = a.rope_cos[(size_t)(pos + tc) * (hd >> 1) + qpair[tn]];
-                            const float sn = a.rope_sin[(size_t)(pos + tc) * (hd >> 1) + qpair[tn]];
-                            const float v0 = (rt & 1) ? other : v, v1 = (rt & 1) ? v : other;
-                            const float r = (rt & 1) ? fadd(fmul(v0, sn), fmul(v1, cs)) : fmul(v0, cs) - fmul(v1, sn);
-                            if (tok_ok) {
-                                if (cb < att) a.q_out[(size_t)t * att + qkcol[tn]] = r;
-                                else a.k_cache[(size_t)qkcol[tn] * a.kv_ld + pos + t] = r;
-                            }
-                        }
-                    } else if (tok_ok && c < a.o) {
-                        if constexpr (EPI == kEpiStore) a.out[(size_t)t * a.o + c] = v;
-                        if constexpr (EPI == kEpiResid) {
-                            // residual add (forward.rs:196-204 / 245-253)
-                            float* xp = a.x + (size_t)t * a.o + c;
-                            *xp = fadd(kResidEarly ? resid[tm][tn][i] : *xp, v);
-                        }
+        for (int i = 0; i < R; i++) {
+            const int t = tl + tok_of(i);
+            const bool tok_ok = t < M;
+            const float v = acc[i];
+            if constexpr (EPI == kEpiQkvRope) {
+                // rope_gguf (util.rs:653-718) on q and k pairs (2j, 2j+1):
+                // the pair partner is the neighbouring lane
+                const float other = dpp_mov<0xB1>(v);
+                // (uniform branches on the tile, as in the initial values)
+                const int att = a.att_dim, kv = a.kv_dim, hd = a.head_size;
+                if (cw >= att + kv) {
+                    if (tok_ok && cw < a.o) a.v_cache[(size_t)(pos + t) * kv + (c - att - kv)] = v;
+                } else {
+                    const int tc = tok_ok ? t : t0;
+                    const float cs = a.rope_cos[(size_t)(pos + tc) * (hd >> 1) + qpair];
+                    const float sn = a.rope_sin[(size_t)(pos + tc) * (hd >> 1) + qpair];
+                    const float v0 = (rt & 1) ? other : v, v1 = (rt & 1) ? v : other;
+                    const float r = (rt & 1) ? fadd(fmul(v0, sn), fmul(v1, cs)) : fmul(v0, cs) - fmul(v1, sn);
+                    if (tok_ok) {
+                        if (cw < att) a.q_out[(size_t)t * att + qkcol] = r;
+                        else a.k_cache[(size_t)qkcol * a.kv_ld + pos + t] = r;
                     }
                 }
+            } else if (tok_ok && c < a.o) {
+                if constexpr (EPI == kEpiStore) a.out[(size_t)t * a.o + c] = v;
+                if constexpr (EPI == kEpiResid) {
+                    // residual add (forward.rs:196-204 / 245-253)
+                    float* xp = a.x + (size_t)t * a.o + c;
+                    *xp = fadd(kResidEarly ? resid[i] : *xp, v);
+                }
+            }
+        }
     }
 
 #endif
@@ -699,24 +606,11 @@ __global__ __launch_bounds__(64 * C::NW) __attribute__((amdgpu_waves_per_eu(C::O
 // ------------------------------------------------------------ dispatch ----
 
 template <int WF, int EPI, class C>
-static size_t gemm_lds() {
-    const size_t stages = (size_t)C::NST * GmStage<WF, C>::bytes;
-    const size_t ex = EPI == kEpiSwiglu && (C::T == 16 || C::WN % 2) ? (size_t)C::TM * (C::TN + 4) * 4 : 0;
-    return std::max(stages, ex);
-}
-
-template <int WF, int EPI, class C>
 static hipError_t launch_gemm_cfg(const GemvArgs& a, int M, hipStream_t st) {
-    const size_t smem = gemm_lds<WF, EPI, C>();
-    if (smem > 65536) {
-        static bool attr_set = false;
-        if (!attr_set) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_gemm<WF, EPI, C>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return e;
-            attr_set = true;
-        }
-    }
+    // the stages, or the sums SwiGLU exchanges
+    constexpr int stages = C::NST * GmStage<WF, C>::bytes, ex = EPI == kEpiSwiglu ? C::TM * (C::TN + 4) * 4 : 0;
+    constexpr int smem = stages > ex ? stages : ex;
+    static_assert(smem <= 64 * 1024 - 64, "dynamic LDS of a launch without the attribute");
     const dim3 grid((a.o + C::TN - 1) / C::TN, (M + C::TM - 1) / C::TM);
     hipLaunchKernelGGL((k_gemm<WF, EPI, C>), grid, dim3(64 * C::NW), smem, st, a, M);
     return hipGetLastError();
@@ -747,16 +641,16 @@ static hipError_t launch_gemm_cfg(const GemvArgs& a, int M, hipStream_t st) {
 // copy (8192 x 8192, M 1000, Wide), the f32 folds alone take 126 us, the
 // MFMAs add 29, the operand reads 26, barriers 16 and the LDS DMA 45 (a DMA
 // instruction occupies the L1 for 64 lane accesses whatever its width).
-using GmOne = GmCfg<16, 1, 1, 1, 1, 4, 3, 2, true>;    // 16 tokens x 16 rows, 1 wavefront
-using GmPair = GmCfg<16, 1, 1, 2, 2, 4, 4, 4>;         // 32 x 32, 4 wavefronts
-using GmQuad = GmCfg<16, 1, 1, 4, 2, 4, 3, 4>;         // 64 x 32, 8 wavefronts
-using GmWide = GmCfg<32, 1, 1, 2, 2, 4, 2, 4>;         // 64 x 64, 4 wavefronts of one 32 x 32 tile
-using GmWide2 = GmCfg<32, 1, 1, 2, 4, 4, 2, 4>;        // 64 x 128, 8 wavefronts: a quarter less traffic per output
+using GmOne = GmCfg<16, 1, 1, 4, 3, 2, true>;    // 16 tokens x 16 rows, 1 wavefront
+using GmPair = GmCfg<16, 2, 2, 4, 4, 4>;         // 32 x 32, 4 wavefronts
+using GmQuad = GmCfg<16, 4, 2, 4, 3, 4>;         // 64 x 32, 8 wavefronts
+using GmWide = GmCfg<32, 2, 2, 4, 2, 4>;         // 64 x 64, 4 wavefronts of one 32 x 32 tile
+using GmWide2 = GmCfg<32, 2, 4, 4, 2, 4>;        // 64 x 128, 8 wavefronts: a quarter less traffic per output
 // SwiGLU needs whole 64-row groups: as many 16-token rows of wavefronts as
 // the batch has
-using GmGate1 = GmCfg<16, 1, 1, 1, 4, 4, 4, 2, true>;  // 16 x 64
-using GmGate2 = GmCfg<16, 1, 1, 2, 4, 4, 4, 4>;        // 32 x 64
-using GmGate4 = GmCfg<16, 1, 1, 4, 4, 4, 3, 4>;        // 64 x 64
+using GmGate1 = GmCfg<16, 1, 4, 4, 4, 2, true>;  // 16 x 64
+using GmGate2 = GmCfg<16, 2, 4, 4, 4, 4>;        // 32 x 64
+using GmGate4 = GmCfg<16, 4, 4, 4, 3, 4>;        // 64 x 64
 
 template <int WF, int EPI>
 static hipError_t launch_gemm_k(const GemvArgs& a, int M, hipStream_t st) {
