@@ -346,7 +346,7 @@ struct yl_session {
     int8_t* gq = nullptr;                // f32-scaled Q8 models: quantized activation row and its scales
     float* gsc = nullptr;
     float* sc = nullptr;                 // attention scores of long contexts [n_heads][ctx]
-    float* psc = nullptr;                // prompt attention scratch (batches of 64+ tokens)
+    float* psc = nullptr;                // prompt attention scratch (the tiled kernels')
     size_t psc_bytes = 0;
     int pseq = 0;                        // seq_len of the prompt call being enqueued
     uint32_t* tokens = nullptr;
@@ -803,7 +803,7 @@ yl_model* model_from_host(HostModel& h, yl_status* st) {
 }
 
 // The prompt attention scratch for `batch` tokens from `start_pos` (kept at
-// the largest size used; prompts below 64 tokens need none).
+// the largest size used; prompts on k_attention need none).
 bool prompt_scratch(yl_session* s, int batch, uint32_t start_pos) {
     s->pseq = (int)start_pos + batch;
     if (!prompt_attn_tiled(batch, s->pseq, s->m->n_heads, s->m->hd)) return true;
@@ -1643,10 +1643,13 @@ namespace {
 // Buffers an attention op call needs beyond its inputs and outputs: the
 // step state (the call's first position), the keys transposed to the
 // kernels' [kv_dim][ld] layout (the caller's are [seq][kv_dim]), and the
-// scores scratch of long decode contexts or of tiled prompt batches.
+// scores scratch of long decode contexts or of tiled prompt batches
+// (sc_bytes; sc_limit is what yl_attention_noalloc holds against its array:
+// the tiled form's scratch for every batch that it can take, so that which
+// calls are refused does not depend on which form runs).
 struct AttnBuffers {
     int ld = 0, kv_dim = 0;
-    size_t kt_bytes = 0, sc_bytes = 0;
+    size_t kt_bytes = 0, sc_bytes = 0, sc_limit = 0;
 };
 
 yl_status attention_plan(const float* out, const float* q, const float* kc, const float* vc, size_t batch,
@@ -1661,9 +1664,9 @@ yl_status attention_plan(const float* out, const float* q, const float* kc, cons
         return YL_ERR_UNSUPPORTED;
     }
     // one token: the decode kernels (as in a decode step); several: the
-    // prompt kernels (one score row per workgroup, or tiled)
-    const bool tiled = prompt_attn_applies((int)batch, (int)seq, (int)hd);
-    if (tiled && hd != 32 && hd != 64 && hd != 128) {
+    // prompt kernels (whole score rows in LDS, or tiled)
+    const bool applies = prompt_attn_applies((int)batch, (int)seq, (int)hd);
+    if (applies && hd != 32 && hd != 64 && hd != 128) {
         set_error("attention: tiled prompt attention needs head_size 32, 64 or 128");
         return YL_ERR_UNSUPPORTED;
     }
@@ -1674,9 +1677,10 @@ yl_status attention_plan(const float* out, const float* q, const float* kc, cons
     B->kv_dim = (int)(n_kv_heads * hd);
     B->ld = ((int)seq + 3) & ~3;
     B->kt_bytes = ((size_t)B->ld * B->kv_dim * 4 + 255) & ~(size_t)255;
-    B->sc_bytes = batch == 1 ? attn_scores_bytes((int)n_heads, (int)seq)
-                  : tiled    ? prompt_attn_bytes((int)n_heads, (int)seq, (int)batch)
+    B->sc_limit = batch == 1 ? attn_scores_bytes((int)n_heads, (int)seq)
+                  : applies  ? prompt_attn_bytes((int)n_heads, (int)seq, (int)batch)
                              : 0;
+    B->sc_bytes = batch == 1 || prompt_attn_tiled((int)batch, (int)seq, (int)n_heads, (int)hd) ? B->sc_limit : 0;
     return YL_OK;
 }
 
@@ -1810,7 +1814,7 @@ yl_status yl_attention_noalloc(float* out, const float* q, const float* kc, cons
     yl_status st = attention_plan(out, q, kc, vc, batch, start_pos, n_heads, n_kv_heads, hd, &B);
     if (st != YL_OK || batch == 0) return st;
     const size_t sc_off = 256 + B.kt_bytes;
-    const size_t need = sc_off + ((B.sc_bytes + 255) & ~(size_t)255);
+    const size_t need = sc_off + ((B.sc_limit + 255) & ~(size_t)255);
     if (need > kNoAllocScratchBytes) {
         set_error("attention_noalloc: the call needs " + std::to_string(need) + " bytes of scratch, more than the " +
                   std::to_string(kNoAllocScratchBytes) + " the library holds per GPU");

@@ -1,7 +1,9 @@
 // yl_pattn.hip -- attention of prompt batches (forward.rs:299-400), tiled.
 //
-// A prompt of B >= 64 tokens attends in three kernels that share every K, V
-// and score tile among 64 query rows.  The arithmetic is the reference's,
+// A prompt large enough to fill the chip with (head, 64-row tile) workgroups
+// (prompt_attn_tiled), or whose score rows do not fit k_attention's LDS,
+// attends in three kernels that share every K, V and score tile among 64
+// query rows.  The arithmetic is the reference's,
 // operation by operation:
 //   score[t][t2] = reduce_add8(8 lane partials over head_size) * scale,
 //     positions past the row's causal bound t1 = pos + t are -1e10;
