@@ -6,8 +6,8 @@ oracle on the same inputs:
 
   SmolLM2-135M Q8_0      256 random prompt ids, then 128 greedy tokens
   Llama-3.2-1B Q8_0      512 random prompt ids, then 256 greedy tokens
-  Llama-3.2-1B Q4_0      512- and 2048-token prompts (int8-MFMA GEMM and the
-                         tiled prompt attention), then greedy steps
+  Llama-3.2-1B Q4_0      512- and 2048-token prompts (int8-MFMA GEMM; the row
+                         and the tiled prompt attention), then greedy steps
   Llama-3-8B mixed       Q4_0 FFN + Q8_0 attention/output, KV cache random-
                          filled to 8192 positions (the oracle cannot prefill
                          8192 tokens of this shape in test time), then
@@ -98,8 +98,9 @@ def test_llama32_1b_q8_full_config(gpu, oracle, model_dir):
 def test_llama32_1b_q4_prefill(gpu, oracle, model_dir, n_prompt, n_steps):
     """Q4_0 weights and activations (reference semantics, weight_type.rs:52-74
     and transformer_llama_gguf.rs:375-410): the prompt's projections run on the
-    int8-MFMA GEMM and its attention on the tiled prompt kernels; then greedy
-    decode steps on the Q4_0 GEMVs."""
+    int8-MFMA GEMM and its attention on four rows per workgroup (512 tokens)
+    or on the tiled kernels (2048); then greedy decode steps on the Q4_0
+    GEMVs."""
     g, o = _models(oracle, model_dir, "llama32_1b_q4")
     _prompt_then_greedy(oracle, g, o, n_prompt, n_steps, seed=n_prompt, compare_steps=n_steps)
 

@@ -36,6 +36,9 @@ CASES = {
     "st_q8_gs128_medium": lambda d: MF.write_safetensors(d, MF.Shape(dim=512, hidden=1536, n_layers=2, n_heads=8,
                                                                      n_kv=2, head_dim=64, ctx=512),
                                                          q8_gs=128, seed=11),
+    # odd block counts (3 and 5 blocks per row)
+    "lmrs_gs32_odd": lambda d: MF.write_lmrs(d, MF.Shape(dim=96, hidden=160, n_heads=3, n_kv=1, head_dim=32), gs=32,
+                                             seed=13),
     # residual rows wide enough that a long prompt's output and down
     # projections take the 64 x 64 tiles (more than 3 M outputs)
     "st_f16_wide": lambda d: MF.write_safetensors(d, MF.Shape(dim=2048, hidden=64, n_layers=1, n_heads=2, n_kv=1,
@@ -65,7 +68,13 @@ def _oracle(path, max_ctx_len=0xFFFFFFFF):
                                                     ("lmrs_gs64", 41, 6), ("lmrs_gs192_medium", 70, 4),
                                                     ("st_q8_medium", 50, 4), ("st_f16_medium", 45, 3),
                                                     ("lmrs_gs32_medium", 37, 5), ("lmrs_gs128", 30, 6),
-                                                    ("st_q8_gs128_medium", 45, 4), ("st_f16_wide", 1530, 1)])
+                                                    ("st_q8_gs128_medium", 45, 4), ("st_f16_wide", 1530, 1),
+                                                    # the tile kernel's last prompt, the GEMM's first ones
+                                                    ("lmrs_gs32", 3, 1), ("lmrs_gs32", 4, 2), ("lmrs_gs32_medium", 15, 1),
+                                                    ("st_q8_gs64", 3, 1), ("st_q8_gs64", 4, 2), ("st_q8_medium", 13, 1),
+                                                    ("lmrs_gs128", 3, 1), ("lmrs_gs128", 4, 2),
+                                                    ("st_q8_gs128_medium", 15, 1), ("lmrs_gs32_odd", 4, 2),
+                                                    ("lmrs_gs32_odd", 21, 2), ("lmrs_gs32_odd", 130, 1)])
 def test_model_matches_oracle(gpu, files, name, prompt_len, steps):
     import yallma3_mini_inference_amd as Y
     path = files(name)

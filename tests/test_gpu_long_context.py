@@ -118,6 +118,19 @@ def test_prompt_row_groups_quantized_head_size_32(gpu, oracle, model_dir, prompt
     assert_bits(gs.value_cache()[:, :prompt_len], os_.value_cache()[:, :prompt_len], "V cache")
 
 
+@pytest.mark.parametrize("name,P", [("tiny_8k", 7300), ("tiny_hd32_long", 8000)])
+def test_prompt_chunk_on_whole_row_tiles(gpu, oracle, model_dir, name, P):
+    """130 tokens past the contexts whose score rows fit k_attention in pairs:
+    the tiled kernels with the quantized output, two whole row tiles and one of
+    two rows, at head sizes 64 and 32."""
+    g, o, _ = _models(oracle, model_dir, name)
+    gs, os_ = g.create_session(), o.create_session()
+    _fill_kv((gs,), os_, P, seed=P)
+    prompt = np.random.default_rng(P).integers(0, o.vocab, 130).astype(np.uint32)
+    assert_bits(g.forward_x(prompt, P, gs), o.forward_x(prompt, P, os_), "prompt")
+    assert_bits(gs.value_cache()[:, P:P + 130], os_.value_cache()[:, P:P + 130], "V cache")
+
+
 def test_split_decode_attention_in_graph(gpu, oracle, model_dir):
     """ctx 8448 (bucket 8448): decode at 5000+ runs k_attn_scores, softmax,
     P.V by lane and the output kernel inside the decode graph with seq well

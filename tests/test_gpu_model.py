@@ -46,8 +46,8 @@ def test_prefill_then_greedy_decode(gpu, oracle, model_dir, name, prompt_len, st
     assert_bits(gs.value_cache()[:, :pos], os_.value_cache()[:, :pos], "V cache")
 
 
-# gate/up tiles of 16, 32 and 64 tokens, their last and first batch, and the
-# GEMV's last
+# gate/up tiles of 16, 32 and 64 tokens, their last and first batch, and
+# shorter prompts (few rows: on the GEMV)
 @pytest.mark.parametrize("name", ["tiny", "tiny_q4", "tiny_pad"])
 @pytest.mark.parametrize("prompt_len", [7, 15, 16, 17, 32, 64, 65])
 def test_prefill_tile_edges(gpu, oracle, model_dir, name, prompt_len):
@@ -57,6 +57,35 @@ def test_prefill_tile_edges(gpu, oracle, model_dir, name, prompt_len):
     assert_bits(g.forward_x(prompt, 0, gs), o.forward_x(prompt, 0, os_), "prefill logits")
     assert_bits(gs.key_cache()[:, :prompt_len], os_.key_cache()[:, :prompt_len], "K cache")
     assert_bits(gs.value_cache()[:, :prompt_len], os_.value_cache()[:, :prompt_len], "V cache")
+
+
+PROMPT_CONFIGS = {
+    # rows by which prompts of 8 to 15 tokens mix the GEMV and the GEMM within
+    # a layer: gate/up on the GEMM from 8 tokens (Q4_0: 14), down from 10, QKV
+    # from 14
+    "rows_16384": dict(dim=2048, hidden=8192, n_layers=2, n_heads=32, n_kv_heads=8, vocab=512, ctx_len=256),
+    # QKV and residual rows on 32 x 32 (430 and 720 tokens) and 64 x 32 tiles
+    "rows_960": dict(dim=576, hidden=64, n_layers=2, n_heads=9, n_kv_heads=3, vocab=512, ctx_len=1024),
+    # QKV, output and down rows on 64 x 128 tiles, whole row tiles of the tiled
+    # attention
+    "rows_3072": dict(dim=2048, hidden=64, n_layers=1, n_heads=32, n_kv_heads=8, vocab=512, ctx_len=4096),
+}
+
+
+@pytest.mark.parametrize("fmt", ["q8", "q4"])
+@pytest.mark.parametrize("name,prompt_lens", [("rows_16384", (7, 8, 9, 10, 12, 13, 14, 15)), ("rows_960", (430, 720)),
+                                              ("rows_3072", (3600,))])
+def test_prompt_projection_tiles(gpu, oracle, tmp_path, fmt, name, prompt_lens):
+    from yallma3_mini_inference_amd import Transformer, synth
+    q = synth.Q4 if fmt == "q4" else synth.Q8
+    path = synth.write(str(tmp_path / "m.gguf"), synth.ModelConfig(**PROMPT_CONFIGS[name], attn_format=q, ffn_format=q, seed=51))
+    g, o = Transformer(path), oracle.Model(path)
+    for n in prompt_lens:
+        prompt = np.random.default_rng(n).integers(0, o.vocab, n).astype(np.uint32)
+        gs, os_ = g.create_session(), o.create_session()
+        assert_bits(g.forward_x(prompt, 0, gs), o.forward_x(prompt, 0, os_), f"{n} tokens")
+        assert_bits(gs.key_cache()[:, :n], os_.key_cache()[:, :n], f"K cache, {n} tokens")
+        assert_bits(gs.value_cache()[:, :n], os_.value_cache()[:, :n], f"V cache, {n} tokens")
 
 
 @pytest.mark.parametrize("name", ["tiny", "tiny_mixed", "tiny_yarn"])

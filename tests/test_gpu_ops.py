@@ -209,7 +209,8 @@ def test_matmul_around_gemv_bound(gpu, oracle, batch, n, o):
 
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("negz", [False, True])
-@pytest.mark.parametrize("batch,n,o", [(96, 512, 384), (2048, 256, 2304)])
+@pytest.mark.parametrize("batch,n,o", [(96, 512, 384), (96, 224, 384), (1100, 224, 400), (1601, 224, 520),
+                                       (2048, 256, 2304), (3000, 224, 2450)])
 def test_matmul_mfma_special_scales(gpu, oracle, fmt, negz, batch, n, o):
     # The GEMM folds the int32-to-f32 convert into an FMA on a biased dot for
     # f16 scales.  That form differs from the reference's only in the sign of
@@ -219,8 +220,9 @@ def test_matmul_mfma_special_scales(gpu, oracle, fmt, negz, batch, n, o):
     # has all-zero activations (every term of its outputs is a signed zero),
     # token 11 two zero blocks.  Initial values are +0 there (the biased form
     # stays exact) or -0 (negz: the workgroup must fall back).  Rows 128..255
-    # hold inf, -inf and NaN scales.  (96, 512, 384) runs 64-token tiles,
-    # (2048, 256, 2304) 128-token tiles.
+    # hold inf, -inf and NaN scales.  Tiles of 16 x 16 (96 tokens), 32 x 32
+    # (1100), 64 x 32 (1601), 64 x 64 (2048) and 64 x 128 (3000); 7 blocks end
+    # in a partial stage and put every other row's scales in half a word.
     from yallma3_mini_inference_amd import QuantizedWeight, WeightFormat, matmul
     rng = np.random.default_rng(5 + fmt + 2 * negz + n)
     nb = n // 32
@@ -429,8 +431,8 @@ def test_attention_decode_chain_lengths(gpu, oracle, seq, nh, nkv, hd):
 
 def test_prompt_attention_nonfinite_v(gpu, oracle):
     # an infinity in V past some rows' causal bound: the reference still adds
-    # p * v there (p = 0), so those rows turn NaN; the tiled kernel must not
-    # skip the masked positions then
+    # p * v there (p = 0), so those rows turn NaN; the kernel must not skip
+    # the masked positions then
     from yallma3_mini_inference_amd import ops
     batch, start, nh, nkv, hd = 96, 10, 4, 2, 64
     rng = np.random.default_rng(96)
@@ -447,16 +449,18 @@ def test_prompt_attention_nonfinite_v(gpu, oracle):
     assert_bits(out[~nan], ref[~nan])
 
 
-def test_tiled_attention_nonfinite_v(gpu, oracle):
-    # the same on a call large enough for the tiled kernels
+@pytest.mark.parametrize("batch", [260, 330])
+def test_tiled_attention_nonfinite_v(gpu, oracle, batch):
+    # the same on four rows per workgroup, and on a call large enough for the
+    # tiled kernels
     from yallma3_mini_inference_amd import ops
-    batch, start, nh, nkv, hd = 260, 10, 64, 4, 64
-    rng = np.random.default_rng(260)
+    start, nh, nkv, hd = 10, 64, 4, 64
+    rng = np.random.default_rng(batch)
     seq = start + batch
     q = rng.normal(0, 1, batch * nh * hd).astype(np.float32)
     kc = rng.normal(0, 1, seq * nkv * hd).astype(np.float32)
     vc = rng.normal(0, 1, seq * nkv * hd).astype(np.float32)
-    vc[(start + 250) * nkv * hd + 3] = np.inf
+    vc[(start + batch - 10) * nkv * hd + 3] = np.inf
     out = ops.attention(q, kc, vc, batch, start, nh, nkv, hd, 0.125)
     ref = oracle.fused_attention(q, kc, vc, seq, batch, nh, nkv, hd, start, nkv * hd, 0.125)
     nan = np.isnan(ref)
@@ -481,28 +485,22 @@ def test_swiglu_quantize(gpu, oracle, hidden, batch, qfmt):
 
 # ends of the row kernels' chunks and passes: less than a workgroup, one, two
 # and four passes, a partial last one; rows without quantized output of any
-# length (elements past the last whole 8 come out zero)
+# length (RMSNorm elements past the last whole 8 come out zero)
 @pytest.mark.parametrize("size,batch,qfmt", [(32, 3, 0), (2080, 2, 1), (4128, 2, 0), (8192, 2, 1), (8, 2, -1),
-                                             (30, 3, -1), (2061, 2, -1)])
+                                             (30, 3, -1), (2061, 2, -1), (3, 2, -1), (1039, 3, -1), (8191, 2, -1)])
 def test_row_kernel_edges(gpu, oracle, size, batch, qfmt):
     from yallma3_mini_inference_amd import WeightFormat, ops, quantize
     rng = np.random.default_rng(size + batch)
     x = rng.normal(0, 2, (batch, size)).astype(np.float32)
     u = rng.normal(0, 1, (batch, size)).astype(np.float32)
     w = rng.normal(1, 0.2, size).astype(np.float32)
-    n8 = size // 8 * 8
-    ref = np.zeros((batch, size), np.float32)
-    for t in range(batch):
-        ref[t] = oracle.rmsnorm(x[t], w, 1e-5) if n8 == size else 0.0
+    ref = np.stack([oracle.rmsnorm(x[t], w, 1e-5) for t in range(batch)])
+    assert np.all(ref[:, size // 8 * 8:] == 0)
     xn, q, s = ops.rmsnorm_quantize(x, w, 1e-5, qfmt)
-    if n8 == size:
-        assert_bits(xn, ref)
-    else:
-        assert np.all(xn[:, n8:] == 0) and np.all(np.isfinite(xn))
+    assert_bits(xn, ref)
     h, hq, hs = ops.swiglu_quantize(x, u, qfmt)
     href = np.stack([oracle.swiglu(x[t], u[t]) for t in range(batch)])
-    if n8 == size:
-        assert_bits(h, href)
+    assert_bits(h, href)
     if qfmt >= 0:
         for got, want in (((q, s), ref), ((hq, hs), href), (quantize(WeightFormat(qfmt), x.ravel()), x)):
             oq, os_ = oracle.quantize(qfmt, want.ravel())

@@ -5,8 +5,8 @@ scores scratch in the library's per-GPU scratch array; its outputs must be
 bit-identical to yl_attention's (which allocates those buffers per call) on
 two calls in a row, the second smaller than the first, for the decode
 kernels (one token: the split path of contexts beyond 4096 with its scores
-scratch, and the single kernel) and the prompt kernels (tiled batches of 64+
-tokens, and the one-row-per-workgroup kernel).  Calls whose buffers exceed
+scratch, and the single kernel) and the prompt kernels (the tiled ones, and
+whole score rows in LDS).  Calls whose buffers exceed
 the array are refused with YL_ERR_RANGE before any work is enqueued.
 """
 import numpy as np
@@ -27,7 +27,8 @@ def _run(lib, fn, q, k, v, batch, start, nh, nkv, hd):
 # (first call, second smaller call): (batch, start_pos, n_heads, n_kv_heads, head_size)
 PAIRS = [
     ((1, 8191, 32, 8, 128), (1, 699, 8, 2, 64)),      # split decode (scores scratch), then one kernel
-    ((70, 30, 8, 2, 64), (20, 10, 8, 2, 64)),         # tiled prompt, then one row per workgroup
+    ((70, 30, 8, 2, 64), (20, 10, 8, 2, 64)),         # prompts on whole score rows
+    ((330, 60, 64, 8, 64), (20, 10, 8, 2, 64)),       # tiled prompt, then whole score rows
     ((1, 5000, 8, 2, 64), (1, 4500, 8, 2, 64)),       # split decode twice, shorter second
 ]
 
