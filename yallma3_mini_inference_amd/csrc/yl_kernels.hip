@@ -38,10 +38,10 @@ typedef unsigned int vu2u __attribute__((ext_vector_type(2), aligned(1)));
 // (Always 256 threads: 2000 rows of 576 6.3 us, now 4.6.)
 template <int QF, int MP>
 __global__ __launch_bounds__(kThreads) void k_rmsnorm(const float* __restrict__ x, const float* __restrict__ w,
-                                                      int dim, float eps, float* xn, int8_t* xq, float* xs) {
+                                                      int dim, float eps, int nt, float* xn, int8_t* xq, float* xs) {
     extern __shared__ __align__(16) float sq[];   // [8][rowq_stride(dim)] squares
     __shared__ float ss_sh;
-    const int t = blockIdx.x, tid = threadIdx.x, nt = blockDim.x, n8 = dim / 8, S = rowq_stride(dim);
+    const int t = blockIdx.x, tid = threadIdx.x, n8 = dim / 8, S = rowq_stride(dim);
     const float* xr = x + (size_t)t * dim;
     float v[MP][8];
 #pragma unroll
@@ -205,10 +205,10 @@ __global__ void k_rope(const float* __restrict__ cos_t, const float* __restrict_
 // Against an element per thread: 1000 rows of 8192 28.7 -> 16.5 us.
 template <int QF>
 __global__ __launch_bounds__(kThreads) void k_swiglu_quant(const float* __restrict__ gate, const float* __restrict__ up,
-                                                           int hidden, float* __restrict__ h_f32,
+                                                           int hidden, int nt, float* __restrict__ h_f32,
                                                            int8_t* __restrict__ hq, float* __restrict__ hs) {
     const int t = blockIdx.y;
-    const int i = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+    const int i = 4 * (blockIdx.x * nt + threadIdx.x);
     const size_t off = (size_t)t * hidden + i;
     float g[4] = {}, u[4] = {}, h[4];
     if (i + 4 <= hidden) {
@@ -393,7 +393,7 @@ static void launch_rmsnorm_q(const float* x, const float* w, int dim, float eps,
     const size_t smem = 8 * (size_t)rowq_stride(dim) * sizeof(float);
     auto k = dim <= 8 * kThreads ? k_rmsnorm<QF, 1> : dim <= 16 * kThreads ? k_rmsnorm<QF, 2> : k_rmsnorm<QF, 4>;
     const int nt = std::min(kThreads, std::max(64, (dim / 8 + 63) & ~63));
-    hipLaunchKernelGGL(k, dim3(batch), dim3(nt), smem, s, x, w, dim, eps, xn, xq, xs);
+    hipLaunchKernelGGL(k, dim3(batch), dim3(nt), smem, s, x, w, dim, eps, nt, xn, xq, xs);
 }
 
 hipError_t launch_rmsnorm(int qfmt, const float* x, const float* w, int dim, float eps, int batch, float* xn,
@@ -431,13 +431,14 @@ hipError_t launch_swiglu_quant(int qfmt, const float* gate, const float* up, int
     // workgroups of equal width, a row of 576 on 192 threads (256: 2000 rows
     // 5.0 us, f32 output only, against 4.5)
     const int chunks = (hidden + 3) / 4, nb = (chunks + kThreads - 1) / kThreads;
-    const dim3 grid(nb, batch), block(((chunks + nb - 1) / nb + 63) & ~63);
+    const int nt = ((chunks + nb - 1) / nb + 63) & ~63;
+    const dim3 grid(nb, batch), block(nt);
     if (qfmt == kQ8)
-        hipLaunchKernelGGL((k_swiglu_quant<kQ8>), grid, block, 0, s, gate, up, hidden, h_f32, hq, hs);
+        hipLaunchKernelGGL((k_swiglu_quant<kQ8>), grid, block, 0, s, gate, up, hidden, nt, h_f32, hq, hs);
     else if (qfmt == kQ4)
-        hipLaunchKernelGGL((k_swiglu_quant<kQ4>), grid, block, 0, s, gate, up, hidden, h_f32, hq, hs);
+        hipLaunchKernelGGL((k_swiglu_quant<kQ4>), grid, block, 0, s, gate, up, hidden, nt, h_f32, hq, hs);
     else
-        hipLaunchKernelGGL((k_swiglu_quant<-1>), grid, block, 0, s, gate, up, hidden, h_f32, hq, hs);
+        hipLaunchKernelGGL((k_swiglu_quant<-1>), grid, block, 0, s, gate, up, hidden, nt, h_f32, hq, hs);
     return hipGetLastError();
 }
 
