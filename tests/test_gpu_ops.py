@@ -378,12 +378,18 @@ def test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd):
 # one, two and four rows per workgroup on either side of their bounds (heads x
 # tokens), below 128, below 256 and from 256 positions; 1 to 5 blocks of 8
 # dimensions per score; one and two dimensions per P.V chain; a last row group
-# of one and of two tokens; whole and partial 16-position runs of the sums
+# of one and of two tokens; whole and partial 16-position runs of the sums; key
+# loads ahead or not on four rows (by workgroups and positions), with 1 to 5
+# blocks
 @pytest.mark.parametrize("batch,start,nh,nkv,hd", [(5, 3, 6, 2, 8), (2, 0, 6, 2, 8), (9, 311, 4, 2, 16), (7, 20, 4, 2, 24),
                                                    (61, 260, 32, 4, 24), (33, 300, 32, 4, 40), (16, 1200, 32, 8, 32),
                                                    (33, 400, 32, 8, 32), (41, 303, 32, 8, 32), (49, 100, 32, 8, 64),
                                                    (57, 0, 32, 8, 64), (33, 10, 64, 8, 32), (33, 200, 64, 8, 8),
-                                                   (40, 239, 32, 8, 64), (40, 240, 32, 8, 64), (57, 256, 9, 3, 64)])
+                                                   (40, 239, 32, 8, 64), (40, 240, 32, 8, 64), (57, 256, 9, 3, 64),
+                                                   (96, 300, 32, 8, 64), (97, 300, 32, 8, 64), (130, 382, 32, 8, 64),
+                                                   (130, 383, 32, 8, 64), (60, 300, 32, 4, 8), (60, 300, 32, 4, 16),
+                                                   (63, 300, 64, 8, 8), (61, 500, 64, 8, 16), (63, 600, 64, 8, 24),
+                                                   (63, 600, 64, 8, 40), (64, 0, 32, 8, 64), (65, 0, 30, 6, 64)])
 def test_attention_row_groups(gpu, oracle, batch, start, nh, nkv, hd):
     test_attention_short_batches(gpu, oracle, batch, start, nh, nkv, hd)
 

@@ -935,7 +935,7 @@ __device__ __forceinline__ float add_row_lanes(float s, float v) {
     return s;
 }
 
-template <int QF, int R, int DD>
+template <int QF, int R, int DD, bool AHEAD>
 __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restrict__ sq,
                                                             const float* __restrict__ kc,
                                                             const float* __restrict__ vc,
@@ -985,7 +985,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
                     for (int j = 0; j < 8; j++) l[r][b][j] = 0.0f;
             vp kn[2][8];
             auto load_k = [&](vp (&k)[8], int s) {
-                const float* ks = kt + (size_t)(8 * s) * kv_ld;
+                const float* ks = kt + (size_t)(8 * (AHEAD ? min(s, n_simd - 1) : s)) * kv_ld;
 #pragma unroll
                 for (int j = 0; j < 8; j++) k[j] = *reinterpret_cast<const vp*>(ks + (size_t)j * kv_ld);
             };
@@ -999,26 +999,41 @@ __global__ __launch_bounds__(kAttnThreads) void k_attention(const float* __restr
                         for (int b = 0; b < PP; b++) l[r][b][j] = fadd(l[r][b][j], fmul(qv, k[j][b]));
                     }
             };
-            load_k(kn[0], 0);
-            if (n_simd > 1) load_k(kn[1], 1);
-            int s = 0;
+            if constexpr (AHEAD) {
+                // every step followed by its buffer's next load (the head's
+                // last block again past its end)
+                load_k(kn[0], 0);
+                load_k(kn[1], 1);
 #pragma unroll 1
-            for (; s + 3 < n_simd; s += 2) {
+                for (int s = 0; s + 1 < n_simd; s += 2) {
+                    step(kn[0], s);
+                    load_k(kn[0], s + 2);
+                    step(kn[1], s + 1);
+                    load_k(kn[1], s + 3);
+                }
+                if (n_simd & 1) step(kn[0], n_simd - 1);
+            } else {
+                load_k(kn[0], 0);
+                if (n_simd > 1) load_k(kn[1], 1);
+                int s = 0;
+#pragma unroll 1
+                for (; s + 3 < n_simd; s += 2) {
+                    step(kn[0], s);
+                    load_k(kn[0], s + 2);
+                    step(kn[1], s + 1);
+                    load_k(kn[1], s + 3);
+                }
+                // the last 1 to 3 (no load past the head: at head size 8 such
+                // re-reads were two loads of three)
+                if (s + 2 < n_simd) {
+                    step(kn[0], s);
+                    load_k(kn[0], s + 2);
+                    step(kn[1], s + 1);
+                    s += 2;
+                }
                 step(kn[0], s);
-                load_k(kn[0], s + 2);
-                step(kn[1], s + 1);
-                load_k(kn[1], s + 3);
+                if (s + 1 < n_simd) step(kn[1], s + 1);
             }
-            // the last 1 to 3 (no load past the head: at head size 8 such
-            // re-reads were two loads of three)
-            if (s + 2 < n_simd) {
-                step(kn[0], s);
-                load_k(kn[0], s + 2);
-                step(kn[1], s + 1);
-                s += 2;
-            }
-            step(kn[0], s);
-            if (s + 1 < n_simd) step(kn[1], s + 1);
 #pragma unroll
             for (int r = 0; r < R; r++)
 #pragma unroll
@@ -1211,7 +1226,7 @@ bool attention_rows4_three_per_cu(int seq_len, int head_size) {
 
 // Rows per workgroup, by rows in all (n = n_heads * batch).  One-row
 // workgroups read K and V once per row but run seven or eight to a CU (64 or
-// 65 registers, against 110 to 127): while all n run at once on short
+// 65 registers, against 96 to 138): while all n run at once on short
 // contexts, one row is the fastest.  From 256 positions the reads weigh more
 // than the latencies and two rows are faster from two one-row workgroups per
 // CU on (four at head size 32, where a row's chains are half as long), four
@@ -1219,6 +1234,8 @@ bool attention_rows4_three_per_cu(int seq_len, int head_size) {
 //   n 1056, head size 64,  183 positions   10.6 / 11.4 / 13.2
 //   n 1536, head size 128, 198             20.1 / 17.1 / 18.6
 //   n 2016, head size 64,  63               8.5 /  9.0 / 10.5
+//   n 2016, head size 32,  63               9.6 /  7.4 /  8.5
+//   n 2016, head size 128, 103             17.2 / 14.0 / 17.7
 //   n 2112, head size 128, 183             24.8 / 28.0 / 20.8
 //   n 288,  head size 64,  1232            24.9 / 28.7 / 36.5
 //   n 1056, head size 64,  1232            45.2 / 40.0 / 41.6
@@ -1228,7 +1245,7 @@ bool attention_rows4_three_per_cu(int seq_len, int head_size) {
 static int attention_rows(int batch, int seq_len, int n_heads, int head_size) {
     const long n = (long)n_heads * batch;
     int rows;
-    if (seq_len < 256) rows = n > 2048 ? 4 : (n > 1792 || (n >= 1536 && seq_len >= 128) ? 2 : 1);
+    if (seq_len < 256) rows = n > 2048 ? 4 : (n > 1792 && (seq_len > 64 || head_size <= 32)) || (n >= 1536 && seq_len >= 128) ? 2 : 1;
     else rows = n >= 1280 ? 4 : (n >= (head_size <= 32 ? 1024 : 512) ? 2 : 1);
     return std::min(rows, attention_rows_fit(seq_len, head_size));
 }
@@ -1243,15 +1260,22 @@ static hipError_t launch_attention_q(const float* sq, const float* kc, const flo
                            n_kv_heads, head_size, scale, aq, as, att_f32);
         return hipGetLastError();
     };
+    // Four rows per workgroup: with the key loads ahead a workgroup takes 138
+    // registers (119 to 127 without) and is 8% faster alone, but three fit a CU
+    // instead of four.  So ahead while all run at once, and on short contexts
+    // where both forms take as many rounds.  Measured in models, us ahead / not:
+    //   9 heads of 64     310 tokens (702 workgroups) 18.3 / 19.8, 350 (792) 30.0 / 21.4
+    //   32 heads of 128   55 from 500 (448) 38.3 / 41.2, 100 (800) 66.6 / 52.9
+    //   16 heads of 64    260 (1040) 27.0 / 29.8, 260 from 500 54.7 / 51.0, 400 (1600) 43.8 / 37.9
+    //   32 heads of 128   260 (2080) 66.6 / 70.9
     const int rows = attention_rows(batch, max_seq, n_heads, head_size);
-    if (head_size <= kAttnThreads / 8) {   // (8 lanes x head_size chains are one round of threads)
-        if (rows == 4) return go(k_attention<QF, 4, 1>, 4);
-        if (rows == 2) return go(k_attention<QF, 2, 1>, 2);
-        return go(k_attention<QF, 1, 1>, 1);
-    }
-    if (rows == 4) return go(k_attention<QF, 4, 2>, 4);
-    if (rows == 2) return go(k_attention<QF, 2, 2>, 2);
-    return go(k_attention<QF, 1, 2>, 1);
+    const long wgs = (long)n_heads * ((batch + 3) / 4);
+    const bool ahead = wgs <= 768 || (max_seq <= 512 && (wgs + 767) / 768 == (wgs + 1023) / 1024);
+    const bool one = head_size <= kAttnThreads / 8;   // 8 lanes x head_size chains are one round of threads
+    if (rows == 4 && ahead) return one ? go(k_attention<QF, 4, 1, true>, 4) : go(k_attention<QF, 4, 2, true>, 4);
+    if (rows == 4) return one ? go(k_attention<QF, 4, 1, false>, 4) : go(k_attention<QF, 4, 2, false>, 4);
+    if (rows == 2) return one ? go(k_attention<QF, 2, 1, false>, 2) : go(k_attention<QF, 2, 2, false>, 2);
+    return one ? go(k_attention<QF, 1, 1, false>, 1) : go(k_attention<QF, 1, 2, false>, 1);
 }
 
 hipError_t launch_attention(const float* sq, const float* kc, const float* vc, const StepState* st, int batch,
