@@ -636,6 +636,10 @@ static hipError_t launch_gemm_cfg(const GemvArgs& a, int M, hipStream_t st) {
 //   3072 x 2048, M 2000                 82.9   53.9   55.0    66.8
 //   8192 x 2048, M 1000                110.8   70.0   68.6    71.9
 //   16384 x 2048, M 2000               450.9  293.2  286.2   290.1
+// Q4_0 and the f32-scaled formats take the same bounds: over 12 shapes of 16 to
+// 2000 tokens Q4_0 is nowhere slower than before, nor are whole prompts of 4 to
+// 1900 tokens with f32 scales (4 layers of the 1B shape, 100 tokens, group size
+// 32 / 64 / 128: 1368 / 1215 / 1245 -> 520 / 495 / 483 us).
 // The large grids stay far from the f32 floor (97 us for the last row at 2
 // cycles per VALU instruction): with parts of the loop taken out in a timing
 // copy (8192 x 8192, M 1000, Wide), the f32 folds alone take 126 us, the
