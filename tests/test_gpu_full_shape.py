@@ -14,9 +14,9 @@ oracle on the same inputs:
                          teacher-forced and greedy decode steps
 
 Bar (forward.rs:120-297, sampler.rs:67-79): logits bit-identical to the
-oracle's at every compared step -- which implies the 1e-3 relative bar the
-north star states, and the largest relative difference is reported -- and
-identical greedy token ids.  Prompt ids are uniform over the vocabulary
+oracle's at every compared step -- which implies the stated 1e-3 relative
+bar, and the largest relative difference is reported -- and identical greedy
+token ids.  Prompt ids are uniform over the vocabulary
 (seeded), as the configurations specify.
 """
 import numpy as np
